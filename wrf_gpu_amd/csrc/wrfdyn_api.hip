@@ -1212,7 +1212,7 @@ int wd_step_noalloc(const wd_grid* grid, const wd_namelist* nl, const wd_state* 
     const double* src;  // host array, or NULL: filled with `value`
     size_t n;
     double value;
-    const double** dst;
+    wd::Met* dst;
   };
   wd::DGrid& g = h.g;
   const Metric metrics[] = {

@@ -30,18 +30,40 @@ constexpr double kCvpm = -(kCp - kRd) / kCp;
 constexpr double kReradius = 1.0 / 6370.0e3;
 constexpr double kPi = 3.141592653589793;
 
+// A metric array: no kernel writes one, so a device read goes through the
+// constant address space.  A read at a wave-uniform index (a vertical metric
+// at the level a wave marches) is then a scalar load; as a plain global read
+// it is a vector load as soon as the kernel has stored anything, and one that
+// waits, in order, for every prefetch issued before it.
+struct Met {
+  const double* p;
+  __host__ __device__ Met& operator=(const double* q) {
+    p = q;
+    return *this;
+  }
+  __host__ __device__ operator const double*() const { return p; }
+  template <class I>
+  __host__ __device__ __forceinline__ double operator[](I k) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return ((const __attribute__((address_space(4))) double*)p)[k];
+#else
+    return p[k];
+#endif
+  }
+};
+
 // Grid + metrics as passed to every kernel (by value, kernarg segment).
 struct DGrid {
   int nx, ny, nz;
   double dx, dy, rdx, rdy;
-  const double *c1h, *c2h, *c1f, *c2f;
-  const double *dnw, *rdnw, *dn, *rdn, *fnm, *fnp;
+  Met c1h, c2h, c1f, c2f;
+  Met dnw, rdnw, dn, rdn, fnm, fnp;
   double cf1, cf2, cf3, cfn, cfn1;
-  const double *msftx, *msfty, *msfux, *msfuy, *msfvx, *msfvy;
-  const double *c3h, *c4h, *c3f, *c4f;  // dry-pressure coefficients (hypsometric_opt 2)
+  Met msftx, msfty, msfux, msfuy, msfvx, msfvy;
+  Met c3h, c4h, c3f, c4f;  // dry-pressure coefficients (hypsometric_opt 2)
   double p_top;
   // Coriolis parameters on mass points (null unless rot): f, e, sina, cosa
-  const double *fcor, *ecor, *sina, *cosa;
+  Met fcor, ecor, sina, cosa;
   int rot;              // 1: f or e nonzero somewhere, the Coriolis terms run
   int hypsometric_opt;  // 2: log-pressure al (WRF calc_p_rho_phi), else linear
   int xcd_remap;  // 1: walk tiles XCD-contiguously (xcd_tile), 0: hardware order

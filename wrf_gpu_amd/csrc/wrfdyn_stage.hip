@@ -1512,8 +1512,7 @@ __global__ void __launch_bounds__(256) k_constk(DGrid g, const double* f, int ki
   const int i = i0 + tx;
   if (i >= ncol) return;
   const bool wl = kind == 2;
-  const double* c1 = wl ? g.c1f : g.c1h;
-  const double* c2 = wl ? g.c2f : g.c2h;
+  const Met c1 = wl ? g.c1f : g.c1h, c2 = wl ? g.c2f : g.c2h;
   const double c1k = c1[k], c2k = c2[k];
   const double dx = g.dx, dy = g.dy, dz = dzp[0];
   const int c = tx + 1;
