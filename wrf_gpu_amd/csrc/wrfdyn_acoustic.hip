@@ -38,7 +38,7 @@ __device__ inline double dpn_ac(const DGrid& g, const double* __restrict__ p, in
 // WET: the state carries moisture (cqu/cqv scale the pressure gradient); dry launches fold them to 1
 template <int BX, int BY, class TT, bool WET>
 __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState s, DWork w,
-                                     double dts) {
+                                     double dts, int first) {
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   // waves overlap by one lane: lanes 1..BX-1 own faces, lane 0 holds the
   // column west of the first owned face
@@ -78,6 +78,17 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     mudf_v = ((-kEmdiv * g.dy) * (s.mudf[cc] - s.mudf[cs])) * msfvx_inv;
     muv = w.muv[i2v(g, j, i)];
   }
+  // The inverse-density perturbation of the last calc_p_rho (core/calc_p_rho.py:
+  // 48-183) is one divide from the new ph work, alt and the column mass, so it
+  // is formed here instead of being stored by the column kernel and read back;
+  // a stage's first substep takes calc_p_rho step 0's column mass.
+  const double muts_c = w.muts[cc], muts_s = w.muts[cs];
+  const double muw_c = first ? w.mu_work0[cc] : muts_c - w.mut[cc];
+  const double muw_s2 = first ? w.mu_work0[cs] : muts_s - w.mut[cs];
+  auto al_at = [&](int k, double alt, double muts, double muw, double ph0, double ph1) {
+    const double safe_mass = safe_pos(g.c1h[k] * muts + g.c2h[k], 1.0e-12);
+    return -(alt * (g.c1h[k] * muw) + g.rdnw[k] * (ph1 - ph0)) / safe_mass;
+  };
   const double* P = w.p;
   // pair sums of p at levels k (carried); psu2/psu1/psu0 = levels k-2, k-1, k
   double pc0 = P[cc], pc1 = P[plane + cc], pc2 = P[2 * plane + cc];
@@ -116,7 +127,6 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     const unsigned ok = (unsigned)k * pl8, ok1 = ok + pl8;
     L.phc1 = ldo(w.ph_work, ok1 + cc8);
     L.altc = ldo(w.alt, ok + cc8);
-    L.alc = ldo(w.al, ok + cc8);
     L.pbc = ldo(w.pb, ok + cc8);
     L.phpc = ldo(w.php, ok + cc8);
     L.pc = ldo(P, ok + cc8);
@@ -130,7 +140,6 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
       if (row_below_outside) {  // rows 1.. of the block take the south column from LDS
         L.phs1 = ldo(w.ph_work, ok1 + cs8);
         L.alts = ldo(w.alt, ok + cs8);
-        L.als = ldo(w.al, ok + cs8);
         L.pbs = ldo(w.pb, ok + cs8);
         L.phps = ldo(w.php, ok + cs8);
         L.ps = ldo(P, ok + cs8);
@@ -186,6 +195,8 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
   for (int k = 0; k < nz; ++k) {
     Lv nxt{};
     if (k + 1 < nz) load(k + 1, nxt);
+    cur.alc = al_at(k, cur.altc, muts_c, muw_c, phc, cur.phc1);
+    if (do_v && row_below_outside) cur.als = al_at(k, cur.alts, muts_s, muw_s2, phs, cur.phs1);
     west(cur);
     south(k, cur);
     // dpn(k+1)
@@ -251,9 +262,9 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
 }
 
 template <int BX, int BY, class TT, bool WET>
-__global__ void __launch_bounds__(BX * BY) k_uv(DGrid g, DState s, DWork w, double dts) {
+__global__ void __launch_bounds__(BX * BY) k_uv(DGrid g, DState s, DWork w, double dts, int first) {
   __shared__ double sh[2][BY][7][BX];
-  b_uv<BX, BY, TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, dts);
+  b_uv<BX, BY, TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, dts, first);
 }
 
 // ---------------------------------------------------------------------------
@@ -739,7 +750,7 @@ __device__ __forceinline__ void b_column(const int tx, const int kt, const unsig
       double p = c2ar[r] * (((alt * (L(E, k) - mu_term * theta_1)) / (safe_mass * safe_t)) - al);
       double ptmp = p;
       p = p + kSmdiv * (p - pm1r[r]);
-      sto(w.al, q, al);
+      if (w.al) sto(w.al, q, al);
       sto(w.p, q, p);
       sto(w.pm1, q, ptmp);
     }
@@ -1207,7 +1218,7 @@ __device__ __forceinline__ void b_column_w(const Blk& B, DGrid g, DNamelist nl, 
         double p = dv.c2a * (((alt * (dv.thw - mu_term * theta_1)) / (safe_mass * safe_t)) - al);
         double ptmp = p;
         p = p + kSmdiv * (p - dv.pm1);
-        sto(w.al, q, al);
+        if (w.al) sto(w.al, q, al);
         sto(w.p, q, p);
         sto(w.pm1, q, ptmp);
       }
@@ -1222,6 +1233,421 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
                                                                                          DState s, DWork w,
                                                                                          double dts, int first) {
   b_column_w<TT>(hw_blk(), g, nl, s, w, dts, first);
+}
+
+// ---------------------------------------------------------------------------
+// Column block: advance_mu_t + advance_w + calc_p_rho of one acoustic substep
+// in one launch, every value by the same operations in the same order as the
+// column march.  A workgroup is one run of 62 columns of a row (64 lanes, one
+// halo lane either side) by KT waves; wave c owns the R consecutive w levels
+// c R .. c R + R - 1 of its lanes' columns and keeps their values in
+// registers from the first load to the last store.  East and west neighbours
+// come from the adjacent lanes (DPP), the levels above and below a wave's own
+// from the adjacent waves (LDS) or a second load.
+//   dmdt and omega: each level's dnw dv, then its omega increment, goes to an
+//     LDS plane; every wave adds up the terms below its own levels itself, in
+//     the column's order, so neither sum passes from wave to wave.
+//   Thomas sweeps: the carried value passes from wave to wave.
+//
+// Why this split: the march pair reads or writes 42 arrays a substep, because
+// each of its sweeps over the levels reads again what the sweep before it had
+// (dvdxi, omega, t_2ave, the phi rhs, the forward-swept w, theta, c2a, alt);
+// with a column's levels spread over the registers of a workgroup each array
+// is read once, 24 in all, and a small grid has thirteen times the waves.
+// Four levels a wave is what 128 VGPRs (four waves per SIMD, one workgroup of
+// up to 16 waves per CU) hold without spilling; 7, 9 and 13 levels a wave at
+// 128, 168 and 256 VGPRs spilled and were slower (433x433x50: 14.8, 17.3 and
+// 14.3 ms a step against 13.3).  At 433x433x50 it moves 2.0 GB in 0.535 ms
+// (3.8 TB/s), bounded by HBM and by the loads that a workgroup cannot issue
+// before its sums; the march pair took 0.659 ms there and 0.144 ms at
+// 64x64x40, where the block takes 0.029.
+// ---------------------------------------------------------------------------
+constexpr int kBlockOwned = 62;   // columns owned per workgroup
+constexpr int kBlockLevels = 4;   // w levels per wave
+constexpr int kBlockExch = 7;     // values per wave and lane of the widest exchange
+
+// Levels per wave with which a grid's columns run as column blocks, 0 where
+// they need more than the 16 waves of a workgroup.
+inline int column_block_levels(int nz) { return nz + 1 <= 16 * kBlockLevels ? kBlockLevels : 0; }
+// LDS of one workgroup (doubles): the two planes of the sums (the first
+// serves the exchanges later) and the carried value of the Thomas sweeps
+__host__ __device__ inline size_t column_block_plane(int nz, int kt) {
+  return (size_t)(nz > kBlockExch * kt ? nz : kBlockExch * kt) * 64;
+}
+inline size_t column_block_lds(int nz, int kt) { return column_block_plane(nz, kt) + (size_t)nz * 64 + 64; }
+
+__device__ __forceinline__ void fence_sched() { __builtin_amdgcn_sched_barrier(0); }
+// The value is computed here: the compiler otherwise sinks an expression to
+// the block of its only use and carries its operands there instead
+__device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
+// Between two phases: nothing moves across, and what depends on v is computed again
+__device__ __forceinline__ void phase_cut(int& v) {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" : "+s"(v));
+}
+
+template <int R, class TT, bool WET>
+__device__ __forceinline__ void b_column_block(const unsigned tile, const int tx, const int c, const int KT, double* lds,
+                                               const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
+                                               double dts, int first) {
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const unsigned nbx = (unsigned)(nx + kBlockOwned - 1) / kBlockOwned;
+  const int i = (int)(tile % nbx) * kBlockOwned + tx - 1;
+  const int j = (int)(tile / nbx);
+  const bool owned = tx >= 1 && tx <= kBlockOwned && i < nx;
+  const int ic = wrapi(i, nx);
+  const unsigned plane = (unsigned)((size_t)ny * nx) * 8u;
+  const unsigned c8 = (unsigned)i2(g, j, ic) * 8u;
+  int f0 = c * R;  // the wave's first w level
+  double* S1 = lds;
+  double* S2 = S1 + column_block_plane(nz, KT);
+  double* carry = S2 + (size_t)nz * 64;
+  const double msfty = ldo(g.msfty, c8);
+  const double eps_p = 1.0 + nl.epssm, eps_m = 1.0 - nl.epssm;
+  const double mut = ldo(w.mut, c8), muts_old = ldo(w.muts, c8);
+  // levels are clamped for the loads, so that every load is in bounds
+  auto mlev = [&](int k) { return k < 0 ? 0 : (k < nz ? k : nz - 1); };
+  auto wlev = [&](int f) { return f < 0 ? 0 : (f <= nz ? f : nz); };
+  auto moff = [&](int k) { return c8 + (unsigned)mlev(k) * plane; };
+  auto woff = [&](int f) { return c8 + (unsigned)wlev(f) * plane; };
+
+  // ---- dvdxi and the horizontal theta flux divergence per mass level ----
+  double dv[R], hf[R], th[R + 2];  // th[r + 1]: theta at level f0 + r
+  {
+    const unsigned uplane = (unsigned)((size_t)ny * (nx + 1)) * 8u, vplane = (unsigned)((size_t)(ny + 1) * nx) * 8u;
+    const unsigned uw8 = (unsigned)i2u(g, j, clampi(i, 0, nx)) * 8u, vs8 = (unsigned)i2v(g, j, ic) * 8u;
+    const unsigned vn8 = (unsigned)i2v(g, j + 1, ic) * 8u;
+    const unsigned cjp = (unsigned)i2(g, wrapi(j + 1, ny), ic) * 8u, cjm = (unsigned)i2(g, wrapi(j - 1, ny), ic) * 8u;
+    const double msftx = ldo(g.msftx, c8);
+    const double muv_n = ldo(w.muv, vn8), muv_s = ldo(w.muv, vs8);
+    const double rmvx_n = 1.0 / ldo(g.msfvx, vn8), rmvx_s = 1.0 / ldo(g.msfvx, vs8);
+    const double muu_w = ldo(w.muu, uw8), msfuy_w = ldo(g.msfuy, uw8);
+    th[0] = ldo(s.theta, moff(f0 - 1));
+    th[R + 1] = ldo(s.theta, moff(f0 + R));
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int k = mlev(f0 + r);
+      const unsigned kv = (unsigned)k * vplane, ku = (unsigned)k * uplane, kp = (unsigned)k * plane;
+      const double uww = ldo(w.u_work, ku + uw8), uw = ldo(s.u, ku + uw8);
+      const double vws = ldo(w.v_work, kv + vs8), vwn = ldo(w.v_work, kv + vn8);
+      const double vs = ldo(s.v, kv + vs8), vn = ldo(s.v, kv + vn8);
+      const double thc = ldo(s.theta, kp + c8), thn = ldo(s.theta, kp + cjp), ths = ldo(s.theta, kp + cjm);
+      const double c1 = g.c1h[k], c2 = g.c2h[k];
+      const double v_n = vwn + ((c1 * muv_n + c2) * vn) * rmvx_n;
+      const double v_s = vws + ((c1 * muv_s + c2) * vs) * rmvx_s;
+      const double u_w = uww + ((c1 * muu_w + c2) * uw) / msfuy_w;
+      const double u_e = wave_shl1(0.0, u_w);
+      dv[r] = (msftx * msfty) * (g.rdy * (v_n - v_s) + g.rdx * (u_e - u_w));
+      if (f0 + r < nz) S1[(size_t)(f0 + r) * 64 + tx] = g.dnw[k] * dv[r];
+      const double t = thc - kT0;
+      const double uwe = wave_shl1(0.0, uww), the = wave_shl1(0.0, thc), thw = wave_shr1(0.0, thc);
+      const double v_flux = vwn * ((thn - kT0) + t) - vws * (t + (ths - kT0));
+      const double u_flux = uwe * ((the - kT0) + t) - uww * (t + (thw - kT0));
+      hf[r] = msftx * ((0.5 * g.rdy) * v_flux + (0.5 * g.rdx) * u_flux);
+      th[r + 1] = thc;
+      pin(hf[r]);
+      pin(dv[r]);
+    }
+  }
+  phase_cut(f0);
+  double thwk[R], tht[R], t2o[R], ww[R + 2];  // ww[r + 1]: omega less the stage's own at level f0 + r
+#pragma unroll
+  for (int r = 0; r < R + 2; ++r) ww[r] = ldo(w.rom, woff(f0 + r - 1));
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const unsigned q = moff(f0 + r);
+    thwk[r] = ldo(w.th_work, q);
+    tht[r] = ldt<TT>(w.tht, q);
+    t2o[r] = first ? 0.0 : ldo(w.t2ave, q);
+  }
+  const double mu_old = ldo(w.mu, c8);
+  const double ww0 = ldo(w.ww, c8), wwtop = ldo(w.ww, woff(nz));
+  phase_cut(f0);
+  __syncthreads();
+
+  // ---- dmdt, the mass updates, the omega increments ----
+  double dmdt = S1[tx];
+  for (int k = 1; k < nz; ++k) dmdt = dmdt + S1[(size_t)k * 64 + tx];
+  const double mu_work_old = muts_old - mut;
+  const double mu_tendency = dmdt + 0.0;
+  const double mu_work = mu_work_old + dts * mu_tendency;
+  const double muts = mut + mu_work;
+  const double muave = 0.5 * (eps_p * mu_work + eps_m * mu_work_old);
+  if (c == 0 && owned) {
+    sto(w.mu, c8, (mu_old - mu_work_old) + mu_work);
+    sto(s.mudf, c8, mu_tendency);
+    sto(w.muts, c8, muts);
+    sto(w.muave, c8, muave);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = mlev(f0 + r);
+    const double incr = (g.dnw[k] * ((g.c1h[k] * dmdt + dv[r]) + g.c1h[k] * 0.0)) / msfty;
+    if (f0 + r < nz) S2[(size_t)(f0 + r) * 64 + tx] = incr;
+  }
+  phase_cut(f0);
+  double c2a[R], alt[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const unsigned q = moff(f0 + r);
+    c2a[r] = ldo(w.c2a, q);
+    alt[r] = ldo(w.alt, q);
+  }
+  __syncthreads();
+  {
+    double wk = ww0;
+    for (int f = 1; f < f0; ++f) wk = wk - S2[(size_t)(f - 1) * 64 + tx];  // omega at f0 - 1
+#pragma unroll
+    for (int r = 0; r < R + 2; ++r) {
+      const int f = f0 + r - 1;
+      if (f >= 1 && f < nz && r > 0) wk = wk - S2[(size_t)(f - 1) * 64 + tx];
+      ww[r] = f < nz ? wk - ww[r] : wwtop;
+      pin(ww[r]);
+    }
+  }
+  if (c == 0 && owned) sto(w.ww, c8, ww[1]);  // level 0 carries to the next substep
+  phase_cut(f0);
+  __syncthreads();  // S2 is free: it holds xp from here on
+
+  // ---- theta update, t_2ave; the theta part of calc_p_rho's bracket; buoyancy ----
+  double buoy[R];
+  double ph1[R + 2];
+#pragma unroll
+  for (int r = 0; r < R + 2; ++r) ph1[r] = ldo(w.ph1t, woff(f0 + r - 1));
+  fence_sched();
+  const double mut_w = muts - mut;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = mlev(f0 + r);
+    const double t = th[r + 1] - kT0;
+    double wd_hi = 0.0, wd_lo = 0.0;
+    if (k + 1 < nz) wd_hi = ww[r + 2] * (g.fnm[k + 1] * (th[r + 2] - kT0) + g.fnp[k + 1] * t);
+    if (k >= 1) wd_lo = ww[r + 1] * (g.fnm[k] * t + g.fnp[k] * (th[r] - kT0));
+    const double tendency = hf[r] + g.rdnw[k] * (wd_hi - wd_lo);
+    const double theta_i = thwk[r] + ((msfty * dts) * tht[r]);
+    const double th_new = theta_i - ((dts * msfty) * tendency);
+    const double mass_h = g.c1h[k] * muts + g.c2h[k];
+    const double half = 0.5 * (eps_p * th_new + eps_m * t2o[r]);
+    const double ttr = kT0 + t;
+    const double t2n = (half + (g.c1h[k] * muave) * kT0) / (mass_h * ttr);
+    buoy[r] = (c2a[r] * alt[r]) * t2n;
+    const double mu_term = g.c1h[k] * mut_w;
+    const double xp = (alt[r] * (th_new - mu_term * t)) / (safe_pos(mass_h, 1.0e-12) * safe_pos(ttr, 1.0e-6));
+    if (f0 + r < nz) {
+      S2[(size_t)(f0 + r) * 64 + tx] = xp;
+    }
+    thwk[r] = th_new;
+    t2o[r] = t2n;
+    pin(buoy[r]);
+    pin(thwk[r]);
+    pin(t2o[r]);
+  }
+  phase_cut(f0);
+
+  double pht[R], rwt[R], phw[R], wold[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    phw[r] = ldo(w.ph_work, woff(f0 + r));
+    wold[r] = ldo(w.w_work, woff(f0 + r));
+    pht[r] = ldt<TT>(w.ph_tend, woff(f0 + r));
+    rwt[r] = ldo(w.rw_tend, woff(f0 + r));
+  }
+  fence_sched();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (owned && f0 + r < nz) {
+      sto(w.th_work, moff(f0 + r), thwk[r]);
+      sto(w.t2ave, moff(f0 + r), t2o[r]);
+    }
+  }
+
+  // ---- phi rhs and the explicit w without its pressure and buoyancy terms ----
+  double rhs[R], wn[R];
+  {
+    const double c05geps = (0.5 * kG) * eps_m;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int f = f0 + r, fc = wlev(f);
+      double rr = dts * (pht[r] + c05geps * wold[r]);
+      if (f < nz && f > 0) {
+        const double wd_f1 = ((0.5 * (ww[r + 2] + ww[r + 1])) * g.rdnw[f]) * (ph1[r + 2] - ph1[r + 1]);
+        const double wd_f = ((0.5 * (ww[r + 1] + ww[r])) * g.rdnw[f - 1]) * (ph1[r + 1] - ph1[r]);
+        const double adv = dts * (g.fnm[f] * wd_f1 + g.fnp[f] * wd_f);
+        rr = rr + (-adv);
+      }
+      const double mass_f = g.c1f[fc] * mut + g.c2f[fc];
+      rr = phw[r] + (msfty * rr) / mass_f;
+      rhs[r] = f == 0 || (f >= nz && nl.top_lid) ? 0.0 : rr;
+      double rw = rwt[r];
+      if (nl.w_damping == 1 && f < nz) {
+        const double safe_mf = safe_pos(mass_f, 1.0e-12);
+        const double vert_cfl = fabs(((ww[r + 1] / safe_mf) * g.rdnw[f]) * dts);
+        const double damp = (((-sgn(wold[r])) * kWAlpha) * (vert_cfl - kWBeta)) * mass_f;
+        rw = rw + (vert_cfl > kWBeta ? damp : 0.0);
+      }
+      wn[r] = wold[r] + dts * rw;
+      pin(wn[r]);
+      pin(rhs[r]);
+    }
+  }
+  phase_cut(f0);
+
+  // ---- the pressure and buoyancy terms of the explicit w, the Thomas rows ----
+  double ca[R], cal[R], cg[R + 1], pm1[R];  // cg[r + 1]: gamma at level f0 + r
+  {
+    auto coef_at = [&](int r) {
+      const int k = mlev(f0 + r);
+      return (c2a[r] * g.rdnw[k]) / safe_pos(g.c1h[k] * mut + g.c2h[k], 1.0e-12);
+    };
+    const double coef_last = coef_at(R - 1);
+#pragma unroll
+    for (int r = 0; r < R + 1; ++r) cg[r] = ldo(w.cgamma, woff(f0 + r - 1));
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      // first substep of a stage: pm1 is the step-0 pressure
+      pm1[r] = ldo(first ? w.p : w.pm1, moff(f0 + r));
+    fence_sched();
+    double* ex = S1 + (size_t)c * kBlockExch * 64 + tx;
+    ex[0 * 64] = rhs[0];
+    ex[1 * 64] = phw[0];
+    ex[2 * 64] = rhs[R - 1];
+    ex[3 * 64] = phw[R - 1];
+    ex[4 * 64] = coef_last;
+    ex[5 * 64] = buoy[R - 1];
+    ex[6 * 64] = c2a[R - 1];
+    __syncthreads();
+    // the first level of the wave above, the last of the wave below
+    const double* up = S1 + (size_t)(c + 1 < KT ? c + 1 : c) * kBlockExch * 64 + tx;
+    const double* dn = S1 + (size_t)(c > 0 ? c - 1 : 0) * kBlockExch * 64 + tx;
+    const double msft_inv = 1.0 / msfty;
+    const double c05dtg = (0.5 * dts) * kG;
+    double cof = (0.5 * dts * kG * (1.0 + nl.epssm));
+    cof = cof * cof;
+    double ta_l = dn[4 * 64] * (eps_p * (rhs[0] - dn[2 * 64]) + eps_m * (phw[0] - dn[3 * 64]));
+    double bl = dn[5 * 64], c2a_m = dn[6 * 64];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int f = f0 + r;
+      const double rhs_u = r + 1 < R ? rhs[r + 1 < R ? r + 1 : r] : up[0 * 64];
+      const double phw_u = r + 1 < R ? phw[r + 1 < R ? r + 1 : r] : up[1 * 64];
+      const double coef = r + 1 < R ? coef_at(r) : coef_last;
+      const double ta_u = coef * (eps_p * (rhs_u - rhs[r]) + eps_m * (phw_u - phw[r]));
+      ca[r] = 0.0;   // the rigid lid's row: w = 0
+      cal[r] = 1.0;
+      if (f >= 1 && f < nz) {
+        const double cq1 = WET ? 1.0 / (1.0 + ldo(w.cqwr, woff(f))) : 1.0;
+        const double termA = ((msft_inv * cq1) * (c05dtg * g.rdn[f])) * (ta_u - ta_l);
+        const double termB = ((dts * kG) * msft_inv) * (g.rdn[f] * (buoy[r] - bl) - (g.c1f[f] * muave));
+        wn[r] = wn[r] + (termA + termB);
+        // the row of calc_coef_w (dynamics/acoustic_wrf.py:783-852): a and
+        // alpha from gamma of the level below, which saves reading them
+        const double mh_m = g.c1h[f - 1] * mut + g.c2h[f - 1], mh = g.c1h[f] * mut + g.c2h[f];
+        const double mf_m = g.c1f[f - 1] * mut + g.c2f[f - 1], mf = g.c1f[f] * mut + g.c2f[f];
+        if (f > 1) ca[r] = (((((-cq1) * cof) * g.rdn[f]) * g.rdnw[f - 1]) * c2a_m) / (mh_m * mf_m);
+        const double b = 1.0 + ((cq1 * cof) * g.rdn[f]) *
+                                   ((g.rdnw[f] * c2a[r]) / (mh * mf) + (g.rdnw[f - 1] * c2a_m) / (mh_m * mf));
+        cal[r] = 1.0 / (b - ca[r] * cg[r]);
+      } else {
+        wn[r] = f == 0 ? ldo(w.wsfc, c8) : 0.0;  // terrain surface w, rigid lid
+      }
+      ta_l = ta_u;
+      bl = buoy[r];
+      c2a_m = c2a[r];
+      pin(wn[r]);
+      pin(ca[r]);
+      pin(cal[r]);
+    }
+  }
+  phase_cut(f0);
+
+  // ---- Thomas sweeps, the carried value from wave to wave ----
+  {
+    for (int q = 0; q < KT; ++q) {
+      if (c == q) {
+        double prev = q > 0 ? carry[tx] : 0.0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (f0 + r > 0) wn[r] = (wn[r] - ca[r] * prev) * cal[r];
+          prev = wn[r];
+        }
+        carry[tx] = prev;
+      }
+      __syncthreads();
+    }
+    for (int q = KT - 1; q >= 0; --q) {
+      if (c == q) {
+        double next = q < KT - 1 ? carry[tx] : 0.0;
+#pragma unroll
+        for (int r = R - 1; r >= 0; --r) {
+          const int f = f0 + r;
+          if (f >= 1 && f < nz) wn[r] = wn[r] - cg[r + 1] * next;
+          next = wn[r];
+        }
+        carry[tx] = next;
+      }
+      __syncthreads();
+    }
+  }
+  phase_cut(f0);
+
+  // ---- damping, the phi finish (rhs becomes the new ph work) ----
+  {
+    const double hdepth = nl.zdamp;
+    const double hbot = ldo(w.ph1t, woff(nz)) / kG - hdepth;
+    const bool damp = nl.damp_opt == 3 && nl.dampcoef > 0.0;
+    fence_sched();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int f = f0 + r;
+      if (f > nz) continue;
+      const unsigned q = c8 + (unsigned)f * plane;
+      if (f == 0) {
+        rhs[r] = ldo(w.ph_work, c8);  // the surface ph work is unchanged
+      } else {
+        if (damp) {
+          const double hk = ldo(w.ph1t, q) / kG;
+          if (hk >= hbot) {  // below the layer the weight is 0 and w passes through
+            const double sn = wd_sin(((0.5 * kPi) * (hk - hbot)) / hdepth);
+            const double dampwt = (dts * nl.dampcoef) * (sn * sn);
+            const double mass_f = g.c1f[f] * mut + g.c2f[f];
+            wn[r] = (wn[r] - (dampwt * mass_f) * ldo(s.w, q)) / (1.0 + dampwt);
+          }
+        }
+        const double mfs = g.c1f[f] * muts + g.c2f[f];
+        rhs[r] = rhs[r] + (((((msfty * 0.5) * dts) * kG) * eps_p) * wn[r]) / mfs;
+        if (owned) sto(w.ph_work, q, rhs[r]);
+      }
+      if (owned) sto(w.w_work, q, wn[r]);
+    }
+  }
+  phase_cut(f0);
+  S1[(size_t)c * 64 + tx] = rhs[0];
+  __syncthreads();
+
+  // ---- calc_p_rho_step ----
+  const double ph_up = S1[(size_t)(c + 1 < KT ? c + 1 : c) * 64 + tx];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = f0 + r;
+    if (k >= nz) continue;
+    const unsigned q = c8 + (unsigned)k * plane;
+    const double safe_mass = safe_pos(g.c1h[k] * muts + g.c2h[k], 1.0e-12);
+    const double mu_term = g.c1h[k] * mut_w;
+    const double phn1 = r + 1 < R ? rhs[r + 1 < R ? r + 1 : r] : ph_up;
+    const double al = -(alt[r] * mu_term + g.rdnw[k] * (phn1 - rhs[r])) / safe_mass;
+    const double ptmp = c2a[r] * (S2[(size_t)k * 64 + tx] - al);
+    if (owned) {
+      sto(w.p, q, ptmp + kSmdiv * (ptmp - pm1[r]));
+      sto(w.pm1, q, ptmp);
+    }
+  }
+}
+
+template <int R, class TT, bool WET>
+__global__ void __launch_bounds__(1024) k_column_block(DGrid g, DNamelist nl, DState s, DWork w, double dts, int first) {
+  extern __shared__ double lds[];
+  b_column_block<R, TT, WET>(tile_id(g), threadIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.y), blockDim.y, lds, g, nl, s,
+                        w, dts, first);
 }
 
 // small_step_finish for w, ph, theta, p and mu (core/small_step_finish.py:22-101)
@@ -1339,6 +1765,9 @@ inline unsigned uv_tiles(const DGrid& g) {
 inline unsigned column_mu_tiles(const DGrid& g) {
   return (unsigned)((g.nx + kMuOwned - 1) / kMuOwned) * (unsigned)((g.ny + kMuRows - 1) / kMuRows);
 }
+inline unsigned column_block_tiles(const DGrid& g) {
+  return (unsigned)((g.nx + kBlockOwned - 1) / kBlockOwned) * (unsigned)g.ny;
+}
 inline unsigned fin_chunks(const DGrid& g) { return (unsigned)((g.nz + kFinChunk - 1) / kFinChunk); }
 
 template <int TX, int KT, int R>
@@ -1377,6 +1806,19 @@ namespace {
 
 hipError_t launch_column_tile(int tile, const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
                               double dts, int first, hipStream_t st, Prof* prof) {
+  if (tile == kColumnMarch && column_block_levels(g.nz) > 0) {
+    const unsigned grid = column_block_tiles(g);
+    const int kt = (g.nz + kBlockLevels) / kBlockLevels;
+    const size_t lds = column_block_lds(g.nz, kt) * sizeof(double);
+    const dim3 block(64, kt);
+    if (nl.mixed)
+      WD_TIMED(prof, KID_COLUMN_BLOCK, st, (k_column_block<kBlockLevels, float, false><<<grid, block, lds, st>>>(g, nl, s, w, dts, first)));
+    else if (w.cqwr)
+      WD_TIMED(prof, KID_COLUMN_BLOCK, st, (k_column_block<kBlockLevels, double, true><<<grid, block, lds, st>>>(g, nl, s, w, dts, first)));
+    else
+      WD_TIMED(prof, KID_COLUMN_BLOCK, st, (k_column_block<kBlockLevels, double, false><<<grid, block, lds, st>>>(g, nl, s, w, dts, first)));
+    return hipGetLastError();
+  }
   if (tile == kColumnMarch) {
     const unsigned bs = 256;
     const size_t C = (size_t)g.ny * g.nx;
@@ -1408,11 +1850,11 @@ hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DS
   constexpr int BX = kUvBx, BY = kUvBy;
   const unsigned uvgrid = uv_tiles(g);
   if (nl.mixed) {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, float, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts)));
+    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, float, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first)));
   } else if (w.cqu) {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, true><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts)));
+    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, true><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first)));
   } else {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts)));
+    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first)));
   }
   // the LDS-tiled kernel has no moisture factor: a moist state runs the column march
   return launch_column_tile(w.cqwr ? kColumnMarch : column_tile, g, nl, s, w, dts, first, st, prof);
@@ -1426,7 +1868,7 @@ hipError_t launch_substep_part(int part, const DGrid& g, const DNamelist& nl, co
   const size_t C = (size_t)g.ny * g.nx;
   if (part == 0) {
     const unsigned uvgrid = uv_tiles(g);
-    k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts);
+    k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first);
   } else if (part == 1) {
     k_column_mu<double><<<column_mu_tiles(g), dim3(64, kMuRows), 0, st>>>(g, nl, s, w, dts, first);
   } else if (part == 2) {
@@ -1452,7 +1894,7 @@ const char* kernel_name(int id) {
       "origin_copy", "k_ruv", "k_rom", "k_prep_col", "k_tend_u", "k_tend_v", "k_tend_w", "k_tend_t",
       "k_prep_2d", "k_prep_faces", "k_prep_u", "k_prep_v", "k_col_setup",
       "k_uv", "k_column", "k_column_mu", "k_column_w", "k_fin_uv", "k_fin_col", "k_diff6", "k_smag", "k_limiter",
-      "k_constk", "k_coriolis", "k_moist", "k_moist_update"};
+      "k_constk", "k_coriolis", "k_moist", "k_moist_update", "k_column_block"};
   return (id >= 0 && id < KID_COUNT) ? names[id] : "";
 }
 

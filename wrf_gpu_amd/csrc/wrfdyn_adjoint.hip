@@ -152,6 +152,7 @@ struct AdjTape {
   void* buf = nullptr;
   size_t bytes = 0;
   TapePtrs p;  // every array carved from buf
+  double* al = nullptr;  // the substeps' inverse-density perturbation, which a plain step does not store
 };
 
 hipError_t adjoint_tape_create(const DGrid& g, const DNamelist& nl, AdjTape** out, size_t* bytes) {
@@ -166,13 +167,15 @@ hipError_t adjoint_tape_create(const DGrid& g, const DNamelist& nl, AdjTape** ou
     delete t;
     return e;
   }
+  const size_t al_bytes = ext_len(g, E_M) * sizeof(double);
   e = hipMemset(t->buf, 0, total);
+  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&t->al), al_bytes);
+  if (e == hipSuccess) e = hipMemset(t->al, 0, al_bytes);
   if (e != hipSuccess) {
-    (void)hipFree(t->buf);
-    delete t;
+    adjoint_tape_destroy(t);
     return e;
   }
-  t->bytes = total;
+  t->bytes = total + al_bytes;
   char* base = static_cast<char*>(t->buf);
   size_t off = 0;
   for (const TapeSlot& x : want) {
@@ -187,6 +190,7 @@ hipError_t adjoint_tape_create(const DGrid& g, const DNamelist& nl, AdjTape** ou
 void adjoint_tape_destroy(AdjTape* t) {
   if (!t) return;
   if (t->buf) (void)hipFree(t->buf);
+  if (t->al) (void)hipFree(t->al);
   delete t;
 }
 
@@ -217,9 +221,11 @@ hipError_t snap_carried(const DGrid& g, const DWork& w, const DState& s, TapePtr
 
 }  // namespace
 
-hipError_t adjoint_large_step(const DGrid& g, const DNamelist& nl, const DWork& w, AdjTape* tape, const DState& start,
-                              const DState& bar_io, hipStream_t st) {
+hipError_t adjoint_large_step(const DGrid& g, const DNamelist& nl, const DWork& work, AdjTape* tape,
+                              const DState& start, const DState& bar_io, hipStream_t st) {
   if (nl.mixed) return hipErrorInvalidValue;
+  DWork w = work;
+  w.al = tape->al;
   TapePtrs& t = tape->p;
   int nsub[3];
   n_boundaries(nl, nsub);

@@ -407,9 +407,9 @@ int workspace_slots(const wd::DGrid& g, const wd::DNamelist& n, bool optional, w
         {&w.vt, V},       {&w.wt, Wn},       {&w.tht, M},      {&w.alt_raw, M},  {&w.al_ls, M},
         {&w.php_ls, M},   {&w.mub, c},       {&w.mut, c},      {&w.muts0, c},    {&w.mu_work0, c},
         {&w.mu, c},       {&w.muts, c},      {&w.muave, c},    {&w.muu, cu},     {&w.muus, cu},
-        {&w.muv, cv},     {&w.muvs, cv},     {&w.u_work, U},   {&w.v_work, V},   {&w.w_work, Wn},
+        {&w.muv, cv},     {&w.muvs, cv},     {&w.wsfc, c},     {&w.u_work, U},   {&w.v_work, V},   {&w.w_work, Wn},
         {&w.th_work, M},  {&w.ph_work, Wn},  {&w.c2a, M},      {&w.alt, M},      {&w.pb, M},
-        {&w.ph1t, Wn},    {&w.php, M},       {&w.p, M},        {&w.al, M},       {&w.pm1, M},
+        {&w.ph1t, Wn},    {&w.php, M},       {&w.p, M},        {&w.pm1, M},
         {&w.rw_tend, Wn}, {&w.ph_tend, Wn},  {&w.ca, Wn},      {&w.calpha, Wn},  {&w.cgamma, Wn},
         {&w.ww, Wn},      {&w.t2ave, M},     {&w.rhs, Wn},     {&w.wfwd, Wn},
     };

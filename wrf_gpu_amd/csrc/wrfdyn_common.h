@@ -106,6 +106,7 @@ struct DWork {
   // prep (2-D)
   double *mub, *mut, *muts0, *mu_work0, *mu, *muts, *muave;
   double *muu, *muus, *muv, *muvs;
+  double *wsfc;  // the terrain surface w of the stage (level 0 of the explicit w)
   // prep (3-D)
   double *u_work, *v_work, *w_work, *th_work, *ph_work;
   double *c2a, *alt, *pb, *ph1t, *php;  // ph1t = origin ph' + base ph (stage constant)

@@ -38,6 +38,7 @@ enum KernelId {
   KID_CORIOLIS,
   KID_MOIST,         // the moisture factors and the species' tendencies
   KID_MOIST_UPDATE,  // the species' large-step update after a stage
+  KID_COLUMN_BLOCK,  // column block: advance_mu_t + advance_w + calc_p_rho
   KID_COUNT
 };
 

@@ -141,7 +141,7 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       b_col_setup<TT, false>(tile, lds, M.g, M.nl, M.s, M.w, S.dts);
       break;
     case PK_UV:
-      b_uv<kUvBx, kUvBy, TT, false>(tile, lds, M.g, M.s, M.w, S.dts);
+      b_uv<kUvBx, kUvBy, TT, false>(tile, lds, M.g, M.s, M.w, S.dts, S.first);
       break;
     case PK_COLUMN_MU:
       b_column_mu<TT>(tile, lds, M.g, M.nl, M.s, M.w, S.dts, S.first);

@@ -886,6 +886,25 @@ __device__ __forceinline__ void b_prep_2d(const Blk& B, DGrid g, DState s, DWork
   w.muts[c] = muts;
   w.mu[c] = mu_cur + mu_work;
   w.muave[c] = 0.0;
+  // terrain surface w (advance_w.py:505-556, level 0 of the explicit w)
+  const int nx = g.nx, ny = g.ny;
+  const int j = (int)(c / (size_t)nx), i = (int)(c % (size_t)nx);
+  const int jn = clampi(j + 1, 0, ny - 1), js = clampi(j - 1, 0, ny - 1);
+  const int ie = clampi(i + 1, 0, nx - 1), iw = clampi(i - 1, 0, nx - 1);
+  auto HT = [&](int jj, int ii) {
+    const size_t q = i2(g, jj, ii);
+    return (s.ph_total[q] - s.ph_pert[q]) / kG;
+  };
+  auto V = [&](int jj) {
+    return (g.cf1 * s.v[iv(g, 0, jj, i)] + g.cf2 * s.v[iv(g, 1, jj, i)]) + g.cf3 * s.v[iv(g, 2, jj, i)];
+  };
+  auto U = [&](int ii) {
+    return (g.cf1 * s.u[iu(g, 0, j, ii)] + g.cf2 * s.u[iu(g, 1, j, ii)]) + g.cf3 * s.u[iu(g, 2, j, ii)];
+  };
+  const double ht = HT(j, i);
+  const double dy_n = HT(jn, i) - ht, dy_s = ht - HT(js, i), dx_e = HT(j, ie) - ht, dx_w = ht - HT(j, iw);
+  w.wsfc[c] = ((g.msfty[c] * 0.5) * g.rdy) * (dy_n * V(j + 1) + dy_s * V(j)) +
+              ((g.msftx[c] * 0.5) * g.rdx) * (dx_e * U(i + 1) + dx_w * U(i));
 }
 
 __global__ void k_prep_2d(DGrid g, DState s, DWork w, int rk_step) {
@@ -1080,7 +1099,7 @@ __device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWor
       double ttr = kT0 + th_ref;
       double safe_t = safe_pos(ttr, 1.0e-6);
       double p = c2a * (((alt_ac * (th_work - mu_term * th_ref)) / (safe_mass * safe_t)) - al);
-      sto(w.al, qk, al);
+      if (w.al) sto(w.al, qk, al);
       sto(w.p, qk, p);
       // pm1 = p and t_2ave = 0 (calc_p_rho_wrf step 0, small_step_prep) are
       // not stored: the stage's first substep reads p for pm1 and starts
