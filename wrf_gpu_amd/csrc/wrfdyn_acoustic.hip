@@ -38,8 +38,9 @@ __device__ inline double dpn_ac(const DGrid& g, const double* __restrict__ p, in
 // WET: the state carries moisture (cqu/cqv scale the pressure gradient); dry launches fold them to 1
 template <int BX, int BY, class TT, bool WET>
 __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState s, DWork w,
-                                     double dts, int first) {
+                                     double dts, int first, int kc) {
   const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   // waves overlap by one lane: lanes 1..BX-1 own faces, lane 0 holds the
   // column west of the first owned face
   const unsigned nbx = (nx + 1 + BX - 2) / (BX - 1);
@@ -90,19 +91,26 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     return -(alt * (g.c1h[k] * muw) + g.rdnw[k] * (ph1 - ph0)) / safe_mass;
   };
   const double* P = w.p;
-  // pair sums of p at levels k (carried); psu2/psu1/psu0 = levels k-2, k-1, k
-  double pc0 = P[cc], pc1 = P[plane + cc], pc2 = P[2 * plane + cc];
-  double pw0 = P[cw], pw1 = P[plane + cw], pw2 = P[2 * plane + cw];
-  double ps0v = P[cs], ps1v = P[plane + cs], ps2v = P[2 * plane + cs];
-  double su0 = pw0 + pc0, su1 = pw1 + pc1, su2 = pw2 + pc2;  // u pair sums, levels 0,1,2
-  double sv0 = ps0v + pc0, sv1 = ps1v + pc1, sv2 = ps2v + pc2;
-  double dpn_u = 0.5 * ((g.cf1 * su0 + g.cf2 * su1) + g.cf3 * su2);  // dpn(0)
-  double dpn_v = 0.5 * ((g.cf1 * sv0 + g.cf2 * sv1) + g.cf3 * sv2);
-  // carried pair sums: cur = level k, prev = k-1, prev2 = k-2
-  double su_cur = su0, su_prev = 0.0, su_prev2 = 0.0;
-  double sv_cur = sv0, sv_prev = 0.0, sv_prev2 = 0.0;
-  double su_next = su1, sv_next = sv1;  // level k+1
-  double phc = w.ph_work[cc], phw = w.ph_work[cw], phs = w.ph_work[cs];  // level k
+  // carried pair sums of p: cur = level k, prev = k-1, prev2 = k-2, next =
+  // k+1; a run that starts at the surface takes levels 1 and 2 for its
+  // bottom face instead of the levels below it
+  auto psum = [&](int k, size_t side) {
+    const size_t o = (size_t)(k < 0 ? 0 : (k < nz ? k : nz - 1)) * plane;
+    return P[o + side] + P[o + cc];
+  };
+  double su_cur = psum(k0, cw), su_prev = psum(k0 ? k0 - 1 : 1, cw), su_prev2 = psum(k0 ? k0 - 2 : 2, cw);
+  double sv_cur = psum(k0, cs), sv_prev = psum(k0 ? k0 - 1 : 1, cs), sv_prev2 = psum(k0 ? k0 - 2 : 2, cs);
+  double su_next = psum(k0 + 1, cw), sv_next = psum(k0 + 1, cs);
+  double dpn_u, dpn_v;  // dpn(k0)
+  if (k0 == 0) {
+    dpn_u = 0.5 * ((g.cf1 * su_cur + g.cf2 * su_prev) + g.cf3 * su_prev2);
+    dpn_v = 0.5 * ((g.cf1 * sv_cur + g.cf2 * sv_prev) + g.cf3 * sv_prev2);
+  } else {
+    dpn_u = 0.5 * (g.fnm[k0] * su_cur + g.fnp[k0] * su_prev);
+    dpn_v = 0.5 * (g.fnm[k0] * sv_cur + g.fnp[k0] * sv_prev);
+  }
+  const size_t o0 = (size_t)k0 * plane;
+  double phc = w.ph_work[o0 + cc], phw = w.ph_work[o0 + cw], phs = w.ph_work[o0 + cs];  // level k
   // Per-level loads, double-buffered: level k+1's loads are issued before
   // level k is computed and stored, so one level of loads is always in flight.
   struct Lv {
@@ -191,10 +199,10 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     L.p2w = wave_shr1(L.p2w, L.p2c);
   };
   Lv cur{};
-  load(0, cur);
-  for (int k = 0; k < nz; ++k) {
+  load(k0, cur);
+  for (int k = k0; k < k1; ++k) {
     Lv nxt{};
-    if (k + 1 < nz) load(k + 1, nxt);
+    if (k + 1 < k1) load(k + 1, nxt);
     cur.alc = al_at(k, cur.altc, muts_c, muw_c, phc, cur.phc1);
     if (do_v && row_below_outside) cur.als = al_at(k, cur.alts, muts_s, muw_s2, phs, cur.phs1);
     west(cur);
@@ -262,9 +270,9 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
 }
 
 template <int BX, int BY, class TT, bool WET>
-__global__ void __launch_bounds__(BX * BY) k_uv(DGrid g, DState s, DWork w, double dts, int first) {
+__global__ void __launch_bounds__(BX * BY) k_uv(DGrid g, DState s, DWork w, double dts, int first, int kc) {
   __shared__ double sh[2][BY][7][BX];
-  b_uv<BX, BY, TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, dts, first);
+  b_uv<BX, BY, TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, dts, first, kc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1263,28 +1271,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 // 64x64x40, where the block takes 0.029.
 // ---------------------------------------------------------------------------
 constexpr int kBlockOwned = 62;   // columns owned per workgroup
-constexpr int kBlockLevels = 4;   // w levels per wave
 constexpr int kBlockExch = 7;     // values per wave and lane of the widest exchange
 
-// Levels per wave with which a grid's columns run as column blocks, 0 where
-// they need more than the 16 waves of a workgroup.
-inline int column_block_levels(int nz) { return nz + 1 <= 16 * kBlockLevels ? kBlockLevels : 0; }
 // LDS of one workgroup (doubles): the two planes of the sums (the first
 // serves the exchanges later) and the carried value of the Thomas sweeps
 __host__ __device__ inline size_t column_block_plane(int nz, int kt) {
   return (size_t)(nz > kBlockExch * kt ? nz : kBlockExch * kt) * 64;
 }
 inline size_t column_block_lds(int nz, int kt) { return column_block_plane(nz, kt) + (size_t)nz * 64 + 64; }
-
-__device__ __forceinline__ void fence_sched() { __builtin_amdgcn_sched_barrier(0); }
-// The value is computed here: the compiler otherwise sinks an expression to
-// the block of its only use and carries its operands there instead
-__device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
-// Between two phases: nothing moves across, and what depends on v is computed again
-__device__ __forceinline__ void phase_cut(int& v) {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" : "+s"(v));
-}
 
 template <int R, class TT, bool WET>
 __device__ __forceinline__ void b_column_block(const unsigned tile, const int tx, const int c, const int KT, double* lds,
@@ -1656,17 +1650,25 @@ __global__ void __launch_bounds__(1024) k_column_block(DGrid g, DNamelist nl, DS
 // thread per column marches up the w levels: the finished ph of levels f-1
 // and f stay in registers for mass level f-1, and the next level's loads are
 // issued before the current level is computed.
-__device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork w) {
+//
+// Where one column a thread leaves the GPU idle, a workgroup is 64 columns by
+// several waves, each marching a run of kc levels (64x64x40: 53 -> 9 us).  The
+// state is updated in place, so a wave reads the old ph of the level below
+// its run before the workgroup's barrier, after which the runs are stored.
+__device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork w, int kc) {
   const size_t ncol = (size_t)g.ny * g.nx;
-  const size_t c = (size_t)tile_id(g, B) * B.bdx + B.tx;
-  if (c >= ncol) return;
+  const size_t cb = (size_t)tile_id(g, B) * B.bdx + B.tx;
+  const bool split = kc <= g.nz;
+  if (!split && cb >= ncol) return;
+  const size_t c = cb < ncol ? cb : ncol - 1;
   const int nz = g.nz;
+  const int f0 = split ? (int)B.ty * kc : 0, f1 = split && f0 + kc < nz + 1 ? f0 + kc : nz + 1;
   const unsigned pl8 = (unsigned)ncol * 8u, c8 = (unsigned)c * 8u;
   const double msfty = g.msfty[c];
   const double muts = w.muts[c], mut = w.mut[c];
   const double mub = w.mub[c], mu_pert_new = w.mu[c];
   const bool hyps2 = g.hypsometric_opt == 2;
-  {
+  if (f0 == 0 && cb < ncol) {
     double mu_base = s.mu_total[c] - s.mu_pert[c];
     s.mu_pert[c] = mu_pert_new;
     s.mu_total[c] = mu_base + mu_pert_new;
@@ -1693,10 +1695,21 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
   };
   Lv cur{}, prev{};
   double pht_prev = 0.0, php_prev = 0.0;  // finished ph total / perturbation at f-1
-  load(0, cur);
-  for (int f = 0; f <= nz; ++f) {
+  if (split) {
+    if (f0 > 0 && f0 < f1) {
+      load(f0 - 1, prev);
+      php_prev = prev.phw + prev.php;
+      pht_prev = (prev.pht - prev.php) + php_prev;
+      pin(php_prev);
+      pin(pht_prev);
+    }
+    __syncthreads();
+    if (cb >= ncol) return;
+  }
+  if (f0 < f1) load(f0, cur);
+  for (int f = f0; f < f1; ++f) {
     Lv nxt{};
-    if (f < nz) load(f + 1, nxt);
+    if (f + 1 < f1) load(f + 1, nxt);
     const unsigned q = c8 + (unsigned)f * pl8;
     // w and ph at level f
     double ms = g.c1f[f] * muts + g.c2f[f];
@@ -1753,7 +1766,10 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
 }
 
 __global__ void __launch_bounds__(256) k_fin_col(DGrid g, DState s, DWork w) {
-  b_fin_col(hw_blk(), g, s, w);
+  b_fin_col(hw_blk(), g, s, w, g.nz + 1);
+}
+__global__ void __launch_bounds__(1024) k_fin_col_runs(DGrid g, DState s, DWork w, int kc) {
+  b_fin_col(hw_blk(), g, s, w, kc);
 }
 
 // Launch grids of the acoustic kernels, which the persistent ensemble step
@@ -1806,9 +1822,9 @@ namespace {
 
 hipError_t launch_column_tile(int tile, const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
                               double dts, int first, hipStream_t st, Prof* prof) {
-  if (tile == kColumnMarch && column_block_levels(g.nz) > 0) {
+  if (tile == kColumnMarch && column_block_waves(g.nz) > 0) {
     const unsigned grid = column_block_tiles(g);
-    const int kt = (g.nz + kBlockLevels) / kBlockLevels;
+    const int kt = column_block_waves(g.nz);
     const size_t lds = column_block_lds(g.nz, kt) * sizeof(double);
     const dim3 block(64, kt);
     if (nl.mixed)
@@ -1848,13 +1864,14 @@ hipError_t launch_column_tile(int tile, const DGrid& g, const DNamelist& nl, con
 hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
                                    double dts, int first, int column_tile, hipStream_t st, Prof* prof) {
   constexpr int BX = kUvBx, BY = kUvBy;
-  const unsigned uvgrid = uv_tiles(g);
+  const int kc = run_levels(uv_tiles(g) * kUvBy, g.nz);
+  const dim3 uvgrid(uv_tiles(g), runs_of(g.nz, kc));
   if (nl.mixed) {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, float, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first)));
+    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, float, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
   } else if (w.cqu) {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, true><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first)));
+    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, true><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
   } else {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first)));
+    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
   }
   // the LDS-tiled kernel has no moisture factor: a moist state runs the column march
   return launch_column_tile(w.cqwr ? kColumnMarch : column_tile, g, nl, s, w, dts, first, st, prof);
@@ -1867,8 +1884,9 @@ hipError_t launch_substep_part(int part, const DGrid& g, const DNamelist& nl, co
   const unsigned bs = 256;
   const size_t C = (size_t)g.ny * g.nx;
   if (part == 0) {
-    const unsigned uvgrid = uv_tiles(g);
-    k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first);
+    const int kc = run_levels(uv_tiles(g) * kUvBy, g.nz);
+    const dim3 uvgrid(uv_tiles(g), runs_of(g.nz, kc));
+    k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc);
   } else if (part == 1) {
     k_column_mu<double><<<column_mu_tiles(g), dim3(64, kMuRows), 0, st>>>(g, nl, s, w, dts, first);
   } else if (part == 2) {
@@ -1885,7 +1903,13 @@ hipError_t launch_stage_finish(const DGrid& g, const DState& s, const DWork& w, 
   const size_t C = (size_t)g.ny * g.nx;
   const unsigned kchunks = fin_chunks(g);
   WD_TIMED(prof, KID_FIN_UV, st, (k_fin_uv<<<dim3(blocks_for(UVcols, bs), kchunks), bs, 0, st>>>(g, s, w)));
-  WD_TIMED(prof, KID_FIN_COL, st, (k_fin_col<<<blocks_for(C, bs), bs, 0, st>>>(g, s, w)));
+  const int kc = column_wave_levels(g, g.nz + 1);
+  if (kc <= g.nz) {
+    const dim3 block(64, runs_of(g.nz + 1, kc));
+    WD_TIMED(prof, KID_FIN_COL, st, (k_fin_col_runs<<<blocks_for(C, 64), block, 0, st>>>(g, s, w, kc)));
+  } else {
+    WD_TIMED(prof, KID_FIN_COL, st, (k_fin_col<<<blocks_for(C, bs), bs, 0, st>>>(g, s, w)));
+  }
   return hipGetLastError();
 }
 

@@ -188,6 +188,42 @@ __device__ inline unsigned tile_id(const DGrid& g, const Blk& b) {
 }
 __device__ inline unsigned tile_id(const DGrid& g) { return tile_id(g, hw_blk()); }
 
+// Levels per workgroup of a k-marching kernel whose launch has `waves` waves
+// when each marches all n levels.  With fewer than kFullWaves of them (two a
+// SIMD) a level's loads wait on each other and nothing else, so the levels are
+// split into runs of at least kRunMin, one row of workgroups (blockIdx.y)
+// each, until the launch has about kRunWaves waves; a run reads the two levels
+// below it again.  Measured, whole steps with and without the runs: 64x64x40
+// (64 waves) 2.49 -> 1.09 ms with runs of 4 levels, 1.05 with 2; 257x257x50
+// (1290 waves) 6.28 -> 5.83 ms at 3072 waves, 5.65 at 6144; at 433x433x50
+// (2930 waves) two runs made k_tend_v 217 -> 236 us and k_tend_w 140 -> 151.
+constexpr unsigned kFullWaves = 2048, kRunWaves = 6144;
+constexpr int kRunMin = 2;
+inline int run_levels(unsigned waves, int n) {
+  if (waves >= kFullWaves) return n;
+  const unsigned runs = kRunWaves / (waves ? waves : 1u);
+  const int kc = (int)((n + runs - 1) / runs);
+  return kc > kRunMin ? kc : kRunMin;
+}
+// Levels per wave of a workgroup of 64 columns whose n levels its waves split
+// between them (at most 16 waves, each with at least one level): n where one
+// column a thread fills the launch.
+inline int column_wave_levels(const DGrid& g, int n) {
+  const int kc = run_levels((unsigned)(((size_t)g.ny * g.nx + 63) / 64), n);
+  return kc >= n ? n : (kc > (n + 15) / 16 ? kc : (n + 15) / 16);
+}
+// Kernels that hold a whole column in one workgroup, kBlockLevels w levels a
+// wave: the waves a grid of nz levels needs, 0 where a workgroup's 16 are too
+// few.
+constexpr int kBlockLevels = 4;
+// The block forms of k_rom and k_col_setup pay while a launch has at most
+// kFewBlocks workgroups (two a CU): 64x64x40 (64 and 128 of them) 23 -> 6.5
+// and 58 -> 32 us, but at 433x433x50 49 -> 77 and 228 -> 613 us, since a
+// workgroup of one row shares no rows.
+constexpr unsigned kFewBlocks = 512;
+inline int column_block_waves(int nz) { return nz + 1 <= 16 * kBlockLevels ? (nz + kBlockLevels) / kBlockLevels : 0; }
+inline unsigned runs_of(int n, int kc) { return (unsigned)((n + kc - 1) / kc); }
+
 inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
 // Loads and stores at a 32-bit byte offset from a wave-uniform base pointer.
@@ -245,6 +281,16 @@ __device__ __forceinline__ double dpp_move(double old, double src) {
   const int lo = __builtin_amdgcn_update_dpp((int)o, (int)v, CTRL, 0xf, 0xf, false);
   const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(v >> 32), CTRL, 0xf, 0xf, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+__device__ __forceinline__ void fence_sched() { __builtin_amdgcn_sched_barrier(0); }
+// The value is computed here: the compiler otherwise sinks an expression to
+// the block of its only use and carries its operands there instead
+__device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
+// Between two phases: nothing moves across, and what depends on v is computed again
+__device__ __forceinline__ void phase_cut(int& v) {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" : "+s"(v));
 }
 
 __device__ inline int clampi(int i, int lo, int hi) { return i < lo ? lo : (i > hi ? hi : i); }

@@ -152,7 +152,7 @@ struct PSeg {
   unsigned vb0;  // the segment's first virtual block in its phase (a multiple of 8)
   unsigned nvb;  // its virtual blocks (256-thread workgroups)
   unsigned gx, gy;  // the standalone launch's grid
-  unsigned aux;     // k_coriolis: its u-face block count
+  unsigned aux;     // k_coriolis: its u-face block count; k-marching kernels: levels per run
 };
 struct PPhase {
   unsigned seg0, nseg;  // segments [seg0, seg0 + nseg), sorted by vb0

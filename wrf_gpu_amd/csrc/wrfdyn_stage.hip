@@ -99,6 +99,46 @@ __global__ void __launch_bounds__(64) k_rom(DGrid g, const double* __restrict__ 
   b_rom(hw_blk(), g, ru, rv, rom);
 }
 
+// The same by a workgroup of 64 columns of a row and one wave per kBlockLevels
+// levels: the divergences go to an LDS plane, from which every wave adds up,
+// in the column's order, what it needs of the two sums.
+__global__ void __launch_bounds__(1024) k_rom_block(DGrid g, const double* __restrict__ ru,
+                                                    const double* __restrict__ rv, double* __restrict__ rom) {
+  extern __shared__ double lds[];
+  constexpr int R = kBlockLevels;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const unsigned nbx = (unsigned)(nx + 63) / 64;
+  const unsigned t = tile_id(g);
+  const int tx = threadIdx.x, k0 = __builtin_amdgcn_readfirstlane(threadIdx.y) * R;
+  const int i = (int)(t % nbx) * 64 + tx, j = (int)(t / nbx);
+  const int ic = i < nx ? i : nx - 1;
+  const int ip = wrapi(ic + 1, nx), jp = wrapi(j + 1, ny);
+  const double msftx = g.msftx[i2(g, j, ic)];
+  double d[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = k0 + r < nz ? k0 + r : nz - 1;
+    d[r] = (g.dnw[k] * msftx) * (g.rdx * (ru[im(g, k, j, ip)] - ru[im(g, k, j, ic)]) +
+                                 g.rdy * (rv[im(g, k, jp, ic)] - rv[im(g, k, j, ic)]));
+    if (k0 + r < nz) lds[(size_t)(k0 + r) * 64 + tx] = d[r];
+  }
+  __syncthreads();
+  double dmdt = 0.0;
+  for (int k = 0; k < nz; ++k) dmdt += lds[(size_t)k * 64 + tx];
+  auto incr_at = [&](int k) { return -((g.dnw[k] * g.c1h[k]) * dmdt) - lds[(size_t)k * 64 + tx]; };
+  double cum = 0.0;
+  for (int k = 0; k < k0; ++k) cum = k == 0 ? incr_at(k) : cum + incr_at(k);
+  if (i >= nx) return;
+  if (k0 == 0) rom[im(g, 0, j, i)] = 0.0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = k0 + r;
+    if (k >= nz) break;
+    cum = k == 0 ? incr_at(k) : cum + incr_at(k);
+    rom[im(g, k + 1, j, i)] = k + 1 < nz ? cum : 0.0;
+  }
+}
+
 // _vertical_flux_div_3 face flux (flux_advection.py:1362-1407) from a column
 // window: qm2..qp1 = q at kf-2 .. kf+1, r = the transport at face kf.
 __device__ inline double vface3(const DGrid& g, int kf, double qm2, double qm1, double q0, double qp1, double r) {
@@ -162,9 +202,10 @@ constexpr int kTendURows = 4;
 template <class TT>
 __device__ __forceinline__ void b_tend_t(const Blk& B, double* lds, DGrid g, DWork w,
                                          const double* __restrict__ th, double qoff, double* dst, const double* d6,
-                                         const double* sm) {
+                                         const double* sm, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   const unsigned nbx = (unsigned)(nx + 61) / 62;
   const unsigned tile = tile_id(g, B);
   const int tx = B.tx, ty = B.ty;
@@ -191,12 +232,25 @@ __device__ __forceinline__ void b_tend_t(const Blk& B, double* lds, DGrid g, DWo
     double ru0, ru1, rv0, rv1;
   };
   // centre-column window of theta (k-1..k+3, raw) and rom (k+1, k+2)
-  double tm1 = 0.0, t0 = ldo(th, c8), tp1 = ldo(th, pl8 + c8), tp2 = ldo(th, 2 * pl8 + c8);
-  double rom1 = ldo(w.rom, pl8 + c8);
-  double ru_n = ldo(w.ru, c8), rv_n = ldo(w.rv, c8);  // own column, one level ahead
+  auto at = [&](int k) { return ldo(th, (unsigned)(k < nz ? k : nz - 1) * pl8 + c8); };
+  double tm1 = 0.0, t0 = at(k0), tp1 = at(k0 + 1), tp2 = at(k0 + 2);
+  double rom1 = ldo(w.rom, (unsigned)(k0 + 1) * pl8 + c8);
+  double ru_n = ldo(w.ru, (unsigned)k0 * pl8 + c8), rv_n = ldo(w.rv, (unsigned)k0 * pl8 + c8);  // one level ahead
   double vf_lo = 0.0;  // vertical face flux at k (0 at the surface)
   double rom0 = 0.0;   // mixed form: rom at face k, and its face interpolant (deviation from level k-1)
   float fdev_lo = 0.0f;
+  if (k0 > 0) {  // a run above the surface: the flux through its lowest face
+    const double tm2 = at(k0 > 1 ? k0 - 2 : 0);
+    tm1 = at(k0 - 1);
+    rom0 = ldo(w.rom, (unsigned)k0 * pl8 + c8);
+    if constexpr (MX) {
+      const double qb = tm1 - qoff;
+      fdev_lo = vface3_dev(g, k0, (float)((tm2 - qoff) - qb), 0.0f, (float)((t0 - qoff) - qb),
+                           (float)((tp1 - qoff) - qb), rom0);
+    } else {
+      vf_lo = vface3(g, k0, tm2 - qoff, tm1 - qoff, t0 - qoff, tp1 - qoff, rom0);
+    }
+  }
   Lv cur{};
   // One mass level.  Level 0 is peeled off the loop, which folds the
   // surface-face branch out of it (measured faster).
@@ -214,7 +268,7 @@ __device__ __forceinline__ void b_tend_t(const Blk& B, double* lds, DGrid g, DWo
     if (!lds_y[4]) cur.rv1 = ldo(w.rv, o + oy[4]);
     cur.ru0 = ru_n;
     cur.rv0 = rv_n;
-    if (k + 1 < nz) {
+    if (k + 1 < k1) {
       ru_n = ldo(w.ru, o + pl8 + c8);
       rv_n = ldo(w.rv, o + pl8 + c8);
     }
@@ -264,26 +318,30 @@ __device__ __forceinline__ void b_tend_t(const Blk& B, double* lds, DGrid g, DWo
     tp2 = tp3;
     rom1 = rom2;
   };
-  level(0);
-  for (int k = 1; k < nz; ++k) level(k);
-
+  int k = k0;
+  if (k0 == 0) {
+    level(0);
+    k = 1;
+  }
+  for (; k < k1; ++k) level(k);
 }
 
 template <class TT>
 __global__ void __launch_bounds__(64 * kTendURows) k_tend_t(DGrid g, DWork w, const double* __restrict__ th,
                                                              double qoff, double* dst, const double* d6,
-                                                             const double* sm) {
+                                                             const double* sm, int kc) {
   __shared__ double sh[2][kTendURows][2][64];
-  b_tend_t<TT>(hw_blk(), &sh[0][0][0][0], g, w, th, qoff, dst, d6, sm);
+  b_tend_t<TT>(hw_blk(), &sh[0][0][0][0], g, w, th, qoff, dst, d6, sm, kc);
 }
 
 // advect_w_flux + _vertical_flux_div_w with a rigid lid
 // (flux_advection.py:1277-1329, 1410-1482) on w levels (nz+1, ny, nx); the
 // transport is _mass_to_full_levels of ru/rv (flux_advection.py:1332-1348).
 template <class TT>
-__device__ __forceinline__ void b_tend_w(const Blk& B, DGrid g, DState s, DWork w) {
+__device__ __forceinline__ void b_tend_w(const Blk& B, DGrid g, DState s, DWork w, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int f0 = (int)B.y * kc, f1 = f0 + kc < nz + 1 ? f0 + kc : nz + 1;  // this block's run of w levels
   const size_t ncol = (size_t)ny * nx;
   const size_t c = (size_t)tile_id(g, B) * B.bdx + B.tx;
   if (c >= ncol) return;
@@ -321,21 +379,41 @@ __device__ __forceinline__ void b_tend_w(const Blk& B, DGrid g, DState s, DWork 
     }
   };
   // centre-column window of w (f-1..f+3) and rom (f, f+1, f+2)
-  double wm1 = 0.0, w0 = ldo(W, c8), wp1 = ldo(W, pl8 + c8), wp2 = ldo(W, 2 * pl8 + c8);
-  double rom0 = ldo(w.rom, c8), rom1 = ldo(w.rom, pl8 + c8);
+  auto at = [&](const double* a, int f) { return ldo(a, (unsigned)(f < nz ? f : nz) * pl8 + c8); };
+  double wm1 = 0.0, w0 = at(W, f0), wp1 = at(W, f0 + 1), wp2 = at(W, f0 + 2);
+  double rom0 = at(w.rom, f0), rom1 = at(w.rom, f0 + 1);
   double vfl_lo = 0.0;  // vflux(f); vflux(0) = 0
   double vf_lo = 0.0;   // mixed form: transport at face f and its interpolant (deviation from w(f-1))
   float fdev_lo = 0.0f;
   double ru0m = 0.0, ru1m = 0.0, rv0m = 0.0, rv1m = 0.0;  // ru/rv at mass level f-1
+  if (f0 > 0) {  // a run above the surface: the flux below its lowest level
+    const unsigned o = (unsigned)(f0 - 1) * pl8;
+    ru0m = ldo(w.ru, o + c8);
+    ru1m = ldo(w.ru, o + cip8);
+    rv0m = ldo(w.rv, o + c8);
+    rv1m = ldo(w.rv, o + cjp8);
+    const double wm2 = at(W, f0 > 1 ? f0 - 2 : 0);
+    wm1 = at(W, f0 - 1);
+    const double vf = 0.5 * (rom0 + at(w.rom, f0 - 1));
+    if constexpr (MX) {
+      if (f0 < nz) {
+        vf_lo = vf;
+        const float dp1 = (float)(w0 - wm1);
+        fdev_lo = f0 == 1 ? 0.5f * dp1 : flux3f((float)(wm2 - wm1), 0.0f, dp1, (float)(wp1 - wm1), sgnf(-vf));
+      }
+    } else if (f0 < nz) {
+      vfl_lo = f0 == 1 ? (vf * 0.5) * (w0 + wm1) : vf * flux3(wm2, wm1, w0, wp1, -vf);
+    }
+  }
   Lv cur{};
-  load(0, cur);
+  load(f0, cur);
   // One w level.  Levels 0 and 1 are peeled off the loop, which folds the
   // surface-face and first-face branches out of it (measured faster).
   auto level = [&](int f) __attribute__((always_inline)) {
     const double wp3 = f + 3 <= nz ? ldo(W, (unsigned)(f + 3) * pl8 + c8) : 0.0;
     const double rom2 = f + 2 <= nz ? ldo(w.rom, (unsigned)(f + 2) * pl8 + c8) : 0.0;
     Lv nxt{};
-    if (f + 1 <= nz) load(f + 1, nxt);
+    if (f + 1 < f1) load(f + 1, nxt);
     auto m2f = [&](double r_f, double r_fm1) {
       if (f == 0) return r_f;
       if (f == nz) return r_fm1;
@@ -402,15 +480,18 @@ __device__ __forceinline__ void b_tend_w(const Blk& B, DGrid g, DState s, DWork 
     }
     cur = nxt;
   };
-  level(0);
-  level(1);
-  for (int f = 2; f <= nz; ++f) level(f);
-
+  int f = f0;
+  if (f0 == 0) {  // kc >= 2: a run from the surface holds both peeled levels
+    level(0);
+    level(1);
+    f = 2;
+  }
+  for (; f < f1; ++f) level(f);
 }
 
 template <class TT>
-__global__ void __launch_bounds__(256) k_tend_w(DGrid g, DState s, DWork w) {
-  b_tend_w<TT>(hw_blk(), g, s, w);
+__global__ void __launch_bounds__(256) k_tend_w(DGrid g, DState s, DWork w, int kc) {
+  b_tend_w<TT>(hw_blk(), g, s, w, kc);
 }
 
 // advect_u_flux (flux_advection.py:1131-1202) + large_step_horizontal_pgf x
@@ -418,9 +499,10 @@ __global__ void __launch_bounds__(256) k_tend_w(DGrid g, DState s, DWork w) {
 // repeats face 0's advection (periodic); the PGF uses edge-padded pairs.
 // WET: the moisture factor cqu scales the PGF; dry launches fold it to 1.
 template <class TT, bool WET>
-__device__ __forceinline__ void b_tend_u(const Blk& B, double* lds, DGrid g, DState s, DWork w) {
+__device__ __forceinline__ void b_tend_u(const Blk& B, double* lds, DGrid g, DState s, DWork w, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   // Blocks of kTendURows rows of one 64-lane wave each; waves overlap by one
   // lane either side (lanes 1..62 own u faces).  Each lane loads its own face
   // (wrapped), its own mass column ia and the PGF's right column; the +-1
@@ -477,7 +559,7 @@ __device__ __forceinline__ void b_tend_u(const Blk& B, double* lds, DGrid g, DSt
   auto shr = [](double v) { return dpp_move<kDppWaveShr1>(0.0, v); };
   auto shl = [](double v) { return dpp_move<kDppWaveShl1>(0.0, v); };
   // ru, rv at the own column, one level ahead (rv goes to LDS before it is used)
-  double ru_n = ldo(w.ru, ca8), rv_n = do_y ? ldo(w.rv, ca8) : 0.0;
+  double ru_n = ldo(w.ru, (unsigned)k0 * pl8 + ca8), rv_n = do_y ? ldo(w.rv, (unsigned)k0 * pl8 + ca8) : 0.0;
   auto load = [&](int k, Lv& L) {
     const unsigned o = (unsigned)k * pl8, ou = (unsigned)k * upl8;
     L.x[0] = ldo(U, ou + ux[0]);
@@ -536,23 +618,36 @@ __device__ __forceinline__ void b_tend_u(const Blk& B, double* lds, DGrid g, DSt
     return 0.5 * (ra + shr(ra));
   };
   const unsigned ua8 = ux[3];
-  double qm1 = 0.0, q0 = ldo(U, ua8), qp1 = ldo(U, upl8 + ua8), qp2 = ldo(U, 2 * upl8 + ua8);
-  double r1 = romq(1);
+  auto at = [&](int k) { return ldo(U, (unsigned)(k < nz ? k : nz - 1) * upl8 + ua8); };
+  double qm1 = 0.0, q0 = at(k0), qp1 = at(k0 + 1), qp2 = at(k0 + 2);
+  double r1 = romq(k0 + 1);
   double vf_lo = 0.0;
   double r0 = 0.0;  // mixed form: face-k transport and interpolant (deviation from level k-1)
   float fdev_lo = 0.0f;
   // p' window at (l, r): level k (p0), k-1 (pm) ; ph' at level k
-  double pl0 = ldo(PP, cl8), pr0 = ldo(PP, cr8), plm = 0.0, prm = 0.0;
-  double phl0 = ldo(s.ph_pert, cl8), phr0 = ldo(s.ph_pert, cr8);
+  const unsigned o0 = (unsigned)k0 * pl8;
+  double pl0 = ldo(PP, o0 + cl8), pr0 = ldo(PP, o0 + cr8), plm = 0.0, prm = 0.0;
+  double phl0 = ldo(s.ph_pert, o0 + cl8), phr0 = ldo(s.ph_pert, o0 + cr8);
   double dpn_k;
-  {
+  if (k0 == 0) {
     const double ps0 = pl0 + pr0;
     const double ps1 = ldo(PP, pl8 + cl8) + ldo(PP, pl8 + cr8);
     const double ps2 = ldo(PP, 2 * pl8 + cl8) + ldo(PP, 2 * pl8 + cr8);
     dpn_k = dpn_ls_bot(g, ps0, ps1, ps2);
+  } else {  // a run above the surface: the flux and dpn of its lowest face
+    plm = ldo(PP, o0 - pl8 + cl8);
+    prm = ldo(PP, o0 - pl8 + cr8);
+    dpn_k = dpn_ls_mid(g, k0, pl0 + pr0, plm + prm);
+    const double qm2 = at(k0 > 1 ? k0 - 2 : 0);
+    qm1 = at(k0 - 1);
+    r0 = romq(k0);
+    if constexpr (MX)
+      fdev_lo = vface3_dev(g, k0, (float)(qm2 - qm1), 0.0f, (float)(q0 - qm1), (float)(qp1 - qm1), r0);
+    else
+      vf_lo = vface3(g, k0, qm2, qm1, q0, qp1, r0);
   }
   Lv cur{};
-  for (int k = 0; k < nz; ++k) {
+  for (int k = k0; k < k1; ++k) {
     const double qp3 = k + 3 < nz ? ldo(U, (unsigned)(k + 3) * upl8 + ua8) : 0.0;
     const double r2 = k + 2 <= nz ? romq(k + 2) : 0.0;
     load(k, cur);
@@ -623,9 +718,9 @@ __device__ __forceinline__ void b_tend_u(const Blk& B, double* lds, DGrid g, DSt
 }
 
 template <class TT, bool WET>
-__global__ void __launch_bounds__(64 * kTendURows) k_tend_u(DGrid g, DState s, DWork w) {
+__global__ void __launch_bounds__(64 * kTendURows) k_tend_u(DGrid g, DState s, DWork w, int kc) {
   __shared__ double sh[2][kTendURows][2][64];
-  b_tend_u<TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w);
+  b_tend_u<TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, kc);
 }
 
 // advect_v_flux (flux_advection.py:1205-1274) + large_step_horizontal_pgf y
@@ -636,9 +731,10 @@ __global__ void __launch_bounds__(64 * kTendURows) k_tend_u(DGrid g, DState s, D
 constexpr int kTendVFields = 9;
 
 template <class TT, bool WET>
-__device__ __forceinline__ void b_tend_v(const Blk& B, double* lds, DGrid g, DState s, DWork w) {
+__device__ __forceinline__ void b_tend_v(const Blk& B, double* lds, DGrid g, DState s, DWork w, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   // Blocks of kTendURows v-face rows of one 64-lane wave each; waves overlap
   // by one lane either side (lanes 1..62 own columns).  Each lane loads its
   // own face (collapsed row ja, column wrapped), its own mass column and the
@@ -698,7 +794,7 @@ __device__ __forceinline__ void b_tend_v(const Blk& B, double* lds, DGrid g, DSt
   };
   auto shl = [](double v) { return dpp_move<kDppWaveShl1>(0.0, v); };
   auto shr = [](double v) { return dpp_move<kDppWaveShr1>(0.0, v); };
-  double ru_n = ldo(w.ru, ca8), rv_n = ldo(w.rv, ca8);  // own column, one level ahead
+  double ru_n = ldo(w.ru, (unsigned)k0 * pl8 + ca8), rv_n = ldo(w.rv, (unsigned)k0 * pl8 + ca8);  // one level ahead
   auto load = [&](int k, Lv& L) {
     const unsigned o = (unsigned)k * pl8, ou = (unsigned)k * upl8;
     L.x[0] = ldo(U, ou + ux[0]);
@@ -779,23 +875,36 @@ __device__ __forceinline__ void b_tend_v(const Blk& B, double* lds, DGrid g, DSt
     return 0.5 * (ldo(w.rom, o + ca8) + ldo(w.rom, o + cjm8));
   };
   const unsigned ua8 = ux[3];
-  double qm1 = 0.0, q0 = ldo(U, ua8), qp1 = ldo(U, upl8 + ua8), qp2 = ldo(U, 2 * upl8 + ua8);
-  double r1 = romq(1);
+  auto at = [&](int k) { return ldo(U, (unsigned)(k < nz ? k : nz - 1) * upl8 + ua8); };
+  double qm1 = 0.0, q0 = at(k0), qp1 = at(k0 + 1), qp2 = at(k0 + 2);
+  double r1 = romq(k0 + 1);
   double vf_lo = 0.0;
   double r0 = 0.0;  // mixed form: face-k transport and interpolant (deviation from level k-1)
   float fdev_lo = 0.0f;
   // p' window at (l, r): level k (p0), k-1 (pm) ; ph' at level k
-  double pl0 = ldo(PP, cl8), pr0 = ldo(PP, cr8), plm = 0.0, prm = 0.0;
-  double phl0 = ldo(s.ph_pert, cl8), phr0 = ldo(s.ph_pert, cr8);
+  const unsigned o0 = (unsigned)k0 * pl8;
+  double pl0 = ldo(PP, o0 + cl8), pr0 = ldo(PP, o0 + cr8), plm = 0.0, prm = 0.0;
+  double phl0 = ldo(s.ph_pert, o0 + cl8), phr0 = ldo(s.ph_pert, o0 + cr8);
   double dpn_k;
-  {
+  if (k0 == 0) {
     const double ps0 = pl0 + pr0;
     const double ps1 = ldo(PP, pl8 + cl8) + ldo(PP, pl8 + cr8);
     const double ps2 = ldo(PP, 2 * pl8 + cl8) + ldo(PP, 2 * pl8 + cr8);
     dpn_k = dpn_ls_bot(g, ps0, ps1, ps2);
+  } else {  // a run above the surface: the flux and dpn of its lowest face
+    plm = ldo(PP, o0 - pl8 + cl8);
+    prm = ldo(PP, o0 - pl8 + cr8);
+    dpn_k = dpn_ls_mid(g, k0, pl0 + pr0, plm + prm);
+    const double qm2 = at(k0 > 1 ? k0 - 2 : 0);
+    qm1 = at(k0 - 1);
+    r0 = romq(k0);
+    if constexpr (MX)
+      fdev_lo = vface3_dev(g, k0, (float)(qm2 - qm1), 0.0f, (float)(q0 - qm1), (float)(qp1 - qm1), r0);
+    else
+      vf_lo = vface3(g, k0, qm2, qm1, q0, qp1, r0);
   }
   Lv cur{};
-  for (int k = 0; k < nz; ++k) {
+  for (int k = k0; k < k1; ++k) {
     const double qp3 = k + 3 < nz ? ldo(U, (unsigned)(k + 3) * upl8 + ua8) : 0.0;
     const double r2 = k + 2 <= nz ? romq(k + 2) : 0.0;
     load(k, cur);
@@ -861,9 +970,9 @@ __device__ __forceinline__ void b_tend_v(const Blk& B, double* lds, DGrid g, DSt
 }
 
 template <class TT, bool WET>
-__global__ void __launch_bounds__(64 * kTendURows) k_tend_v(DGrid g, DState s, DWork w) {
+__global__ void __launch_bounds__(64 * kTendURows) k_tend_v(DGrid g, DState s, DWork w, int kc) {
   __shared__ double sh[2][kTendURows][kTendVFields][64];
-  b_tend_v<TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w);
+  b_tend_v<TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, kc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1004,7 +1113,7 @@ __global__ void __launch_bounds__(256) k_prep_v(DGrid g, DState s, DWork w) {
 //                c2a, php and calc_p_rho_wrf step 0 al, p
 //                (core/calc_p_rho.py:48-139)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWork w) {
+__device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWork w, int kc) {
   const size_t ncol = (size_t)g.ny * g.nx;
   const size_t c = (size_t)tile_id(g, B) * B.bdx + B.tx;
   if (c >= ncol) return;
@@ -1034,11 +1143,13 @@ __device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWor
       L.th0 = ldo(w.th0, q);
     }
   };
+  const int f0 = (int)B.y * kc, f1 = f0 + kc < nz + 1 ? f0 + kc : nz + 1;  // this block's run of w levels
   Lv cur{}, prev{};
-  load(0, cur);
-  for (int f = 0; f <= nz; ++f) {
+  if (f0 > 0) load(f0 - 1, prev);
+  load(f0, cur);
+  for (int f = f0; f < f1; ++f) {
     Lv nxt{};
-    if (f < nz) load(f + 1, nxt);
+    if (f + 1 < f1) load(f + 1, nxt);
     const unsigned q = c8 + (unsigned)f * pl8;
     {  // w level f
       double mref = g.c1f[f] * muts0 + g.c2f[f];
@@ -1110,8 +1221,8 @@ __device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWor
   }
 }
 
-__global__ void __launch_bounds__(256) k_prep_col(DGrid g, DState s, DWork w) {
-  b_prep_col(hw_blk(), g, s, w);
+__global__ void __launch_bounds__(256) k_prep_col(DGrid g, DState s, DWork w, int kc) {
+  b_prep_col(hw_blk(), g, s, w, kc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1365,6 +1476,187 @@ __device__ __forceinline__ void b_col_setup(const Blk& B, double* lds, DGrid g, 
   sto(w.ca, qt, a_top);
   sto(w.calpha, qt, 1.0 / (b_top - a_top * gamma_prev));
   sto(w.cgamma, qt, 0.0);
+}
+
+// The same column setup by a workgroup of 62 columns of a row (one halo lane
+// either side) and one wave per kBlockLevels levels: each wave forms its
+// levels' tendencies and matrix rows from its own loads, and the gamma
+// recurrence passes from wave to wave.  One wave more per four levels is what
+// a small grid lacks.
+template <class TT, bool WET>
+__global__ void __launch_bounds__(1024) k_col_setup_block(DGrid g, DNamelist nl, DState s, DWork w, double dts) {
+  __shared__ double carry[64];
+  constexpr int R = kBlockLevels;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const unsigned nbx = (unsigned)(nx + kColOwned - 1) / kColOwned;
+  const unsigned tile = tile_id(g);
+  const int tx = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y), KT = blockDim.y;
+  const int i = (int)(tile % nbx) * kColOwned + tx - 1;
+  const int j = (int)(tile / nbx);
+  const bool owned = tx >= 1 && tx <= kColOwned && i < nx;
+  const int ic = wrapi(i, nx), f0 = wave * R;
+  const size_t c = i2(g, j, ic);
+  const unsigned pl8 = (unsigned)((size_t)ny * nx) * 8u, c8 = (unsigned)c * 8u;
+  const unsigned upl8 = (unsigned)((size_t)ny * (nx + 1)) * 8u, vpl8 = (unsigned)((size_t)(ny + 1) * nx) * 8u;
+  const size_t fuw = i2u(g, j, clampi(i, 0, nx)), fvs = i2v(g, j, ic), fvn = i2v(g, j + 1, ic);
+  const unsigned uw8 = (unsigned)fuw * 8u, vs8 = (unsigned)fvs * 8u, vn8 = (unsigned)fvn * 8u;
+  const unsigned cjp8 = (unsigned)i2(g, wrapi(j + 1, ny), ic) * 8u, cjm8 = (unsigned)i2(g, wrapi(j - 1, ny), ic) * 8u;
+  const double msfty = g.msfty[c], msft_inv = 1.0 / msfty;
+  const double mut = w.mut[c], mub = w.mub[c], mu_p = mut - mub;
+  const double mxy = g.msftx[c] / msfty;
+  const double e_c = g.rot ? g.ecor[c] : 0.0, cosa_c = g.rot ? g.cosa[c] : 1.0, sina_c = g.rot ? g.sina[c] : 0.0;
+  const double muu_w = w.muu[fuw], msfuy_w = g.msfuy[fuw];
+  const double muu_e = dpp_move<kDppWaveShl1>(0.0, muu_w);
+  const double muv_s = w.muv[fvs], muv_n = w.muv[fvn], msfvx_s = g.msfvx[fvs], msfvx_n = g.msfvx[fvn];
+  double cof = (0.5 * dts * kG * (1.0 + nl.epssm));
+  cof = cof * cof;
+  const double lid_flag = nl.top_lid ? 0.0 : 1.0;
+  auto MH = [&](int k) { return g.c1h[k] * mut + g.c2h[k]; };
+  auto MF = [&](int k) { return g.c1f[k] * mut + g.c2f[k]; };
+  auto PHT = [&](double pert, double total) { return pert + (total - pert); };
+  // the wave's mass levels f0 - 1 .. f0 + R - 1, clamped into the column
+  double uw[R + 1], vs[R + 1], vn[R + 1], pp[R + 1], c2a[R + 1];
+  double rom[R + 2], pht[R + 2], pn[R], ps[R], wt[R], ww[R], cqr[R + 1];
+  auto load_m = [&](int r) {
+    const int k = clampi(f0 + r - 1, 0, nz - 1);
+    uw[r] = ldo(s.u, (unsigned)k * upl8 + uw8);
+    vs[r] = ldo(s.v, (unsigned)k * vpl8 + vs8);
+    vn[r] = ldo(s.v, (unsigned)k * vpl8 + vn8);
+    pp[r] = ldo(s.p_pert, (unsigned)k * pl8 + c8);
+    c2a[r] = ldo(w.c2a, (unsigned)k * pl8 + c8);
+    cqr[r] = WET ? ldo(w.cqwr, (unsigned)k * pl8 + c8) : 0.0;
+  };
+  auto load_w = [&](int r) {
+    const unsigned q = (unsigned)clampi(f0 + r - 1, 0, nz) * pl8 + c8;
+    rom[r] = ldo(w.rom, q);
+    pht[r] = PHT(ldo(s.ph_pert, q), ldo(s.ph_total, q));
+  };
+  auto load_f = [&](int r) {
+    const unsigned o = (unsigned)clampi(f0 + r, 0, nz) * pl8;
+    pn[r] = PHT(ldo(s.ph_pert, o + cjp8), ldo(s.ph_total, o + cjp8));
+    ps[r] = PHT(ldo(s.ph_pert, o + cjm8), ldo(s.ph_total, o + cjm8));
+    wt[r] = ldt<TT>(w.wt, o + c8);
+    ww[r] = ldo(s.w, o + c8);
+  };
+  load_m(0);
+  load_w(0);
+  load_w(1);
+  load_m(1);
+  load_w(2);
+  load_f(0);
+  // curvature pieces at mass level k: ru, u, rv, v averaged to the column
+  struct Cv {
+    double ru_m, u_m, rv_m, v_m;
+  };
+  auto curv_at = [&](int r) {
+    const int k = clampi(f0 + r - 1, 0, nz - 1);
+    Cv x;
+    const double ru_l = ((g.c1h[k] * muu_w + g.c2h[k]) * uw[r]) / msfuy_w;
+    const double ru_r = dpp_move<kDppWaveShl1>(0.0, ru_l), ue = dpp_move<kDppWaveShl1>(0.0, uw[r]);
+    x.ru_m = 0.5 * (ru_l + ru_r);
+    x.u_m = 0.5 * (uw[r] + ue);
+    const double rv_s = ((g.c1h[k] * muv_s + g.c2h[k]) * vs[r]) / msfvx_s;
+    const double rv_n = ((g.c1h[k] * muv_n + g.c2h[k]) * vn[r]) / msfvx_n;
+    x.rv_m = 0.5 * (rv_s + rv_n);
+    x.v_m = 0.5 * (vs[r] + vn[r]);
+    return x;
+  };
+  Cv cv_m = curv_at(0);
+  double ak[R], bk[R], ck[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int f = f0 + r;
+    if (r + 1 < R) {  // one level ahead
+      load_m(r + 2 < R + 1 ? r + 2 : R);
+      load_w(r + 3 < R + 2 ? r + 3 : R + 1);
+      load_f(r + 1 < R ? r + 1 : r);
+    }
+    fence_sched();
+    const Cv cv0 = curv_at(r + 1);
+    const unsigned q = c8 + (unsigned)f * pl8;
+    const double ue = dpp_move<kDppWaveShl1>(0.0, uw[r + 1]), ue_m = dpp_move<kDppWaveShl1>(0.0, uw[r]);
+    const double pht_e = dpp_move<kDppWaveShl1>(0.0, pht[r + 1]), pht_w = dpp_move<kDppWaveShr1>(0.0, pht[r + 1]);
+    ak[r] = 0.0;
+    bk[r] = 1.0;
+    ck[r] = 0.0;
+    if (f == 0) {
+      if (owned) {
+        sto(w.rw_tend, q, 0.0 + wt[r]);
+        stt<TT>(w.ph_tend, q, 0.0);
+      }
+    } else if (f < nz) {
+      const double cq1 = WET ? 1.0 / (1.0 + cqr[r + 1]) : 1.0, cq2 = WET ? cqr[r + 1] * cq1 : 0.0;
+      {
+        double rw = (msft_inv * kG) *
+                    (((cq1 * g.rdn[f]) * (pp[r + 1] - pp[r]) - g.c1f[f] * mu_p) - cq2 * (g.c1f[f] * mub + g.c2f[f]));
+        rw = rw + wt[r];
+        const double ru_f = g.fnm[f] * cv0.ru_m + g.fnp[f] * cv_m.ru_m;
+        const double u_f = g.fnm[f] * cv0.u_m + g.fnp[f] * cv_m.u_m;
+        const double rv_f = g.fnm[f] * cv0.rv_m + g.fnp[f] * cv_m.rv_m;
+        const double v_f = g.fnm[f] * cv0.v_m + g.fnp[f] * cv_m.v_m;
+        const double curv = kReradius * (ru_f * u_f + (mxy * rv_f) * v_f);
+        const double cor = g.rot ? e_c * (cosa_c * ru_f - (mxy * sina_c) * rv_f) : 0.0;
+        if (owned) sto(w.rw_tend, q, rw + (cor + curv));
+      }
+      {
+        const double wd_f = ((0.5 * (rom[r + 2] + rom[r + 1])) * g.rdnw[f]) * (pht[r + 2] - pht[r + 1]);
+        const double wd_fm = ((0.5 * (rom[r + 1] + rom[r])) * g.rdnw[f - 1]) * (pht[r + 1] - pht[r]);
+        const double term3 = g.fnm[f] * wd_f + g.fnp[f] * wd_fm;
+        double t = -term3;
+        const double mass_f = g.c1f[f] * mut + g.c2f[f];
+        t = t + ((mass_f * kG) * ww[r]) * msft_inv;
+        const double pti = pht[r + 1];
+        const double dn_ = pn[r] - pti, ds_ = pti - ps[r];
+        const double mvn = g.c1f[f] * muv_n + g.c2f[f], mvs = g.c1f[f] * muv_s + g.c2f[f];
+        const double fy = (mvn * (vn[r + 1] + vn[r])) * dn_ + (mvs * (vs[r + 1] + vs[r])) * ds_;
+        t = t + (-((0.25 * g.rdy) * msft_inv)) * fy;
+        const double de_ = pht_e - pti, dw_ = pti - pht_w;
+        const double mue = g.c1f[f] * muu_e + g.c2f[f], muw = g.c1f[f] * muu_w + g.c2f[f];
+        const double fx = (mue * (ue + ue_m)) * de_ + (muw * (uw[r + 1] + uw[r])) * dw_;
+        t = t + (-((0.25 * g.rdx) * msft_inv)) * fx;
+        if (owned) stt<TT>(w.ph_tend, q, t);
+      }
+      if (f > 1) ak[r] = (((((-cq1) * cof) * g.rdn[f]) * g.rdnw[f - 1]) * c2a[r]) / (MH(f - 1) * MF(f - 1));
+      const double du = MH(f) * MF(f), dl = MH(f - 1) * MF(f), dc = MH(f) * MF(f + 1);
+      bk[r] = 1.0 + ((cq1 * cof) * g.rdn[f]) * ((g.rdnw[f] * c2a[r + 1]) / du + (g.rdnw[f - 1] * c2a[r]) / dl);
+      ck[r] = (((((-cq1) * cof) * g.rdn[f]) * g.rdnw[f]) * c2a[r + 1]) / dc;
+    } else if (f == nz) {  // the raw cqw of face nz - 1
+      const double cq1 = WET ? 1.0 / (1.0 + cqr[r]) : 1.0, cq2 = WET ? cqr[r] * cq1 : 0.0;
+      const double rwt = (msft_inv * kG) * (((((cq1 * 2.0) * g.rdnw[nz - 1]) * (-pp[r])) - g.c1f[nz] * mu_p) -
+                                            cq2 * (g.c1f[nz] * mub + g.c2f[nz]));
+      const double r2 = g.rdnw[nz - 1] * g.rdnw[nz - 1];
+      ak[r] = ((((-2.0 * cof) * r2) * c2a[r]) * lid_flag) / (MH(nz - 1) * MF(nz - 1));
+      bk[r] = 1.0 + (((2.0 * cof) * r2) * c2a[r]) / (MH(nz - 1) * MF(nz));
+      if (owned) {
+        sto(w.rw_tend, q, rwt + wt[r]);
+        stt<TT>(w.ph_tend, q, 0.0);
+      }
+    }
+    cv_m = cv0;
+    pin(ak[r]);
+    pin(bk[r]);
+    pin(ck[r]);
+  }
+  for (int q = 0; q < KT; ++q) {
+    if (wave == q) {
+      double gamma = q > 0 ? carry[tx] : 0.0;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int f = f0 + r;
+        if (f > nz) break;
+        const unsigned o = c8 + (unsigned)f * pl8;
+        const double al = f == 0 ? 1.0 : 1.0 / (bk[r] - ak[r] * gamma);
+        gamma = f == 0 ? 0.0 : ck[r] * al;
+        if (owned) {
+          sto(w.cgamma, o, f < nz ? gamma : 0.0);
+          sto(w.ca, o, ak[r]);
+          sto(w.calpha, o, al);
+        }
+      }
+      carry[tx] = gamma;
+    }
+    __syncthreads();
+  }
 }
 
 template <class TT, bool WET>
@@ -2126,6 +2418,7 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
   const size_t C = (size_t)g.ny * g.nx;
   const size_t F = (size_t)g.ny * (g.nx + 1) + (size_t)(g.ny + 1) * g.nx;
   const unsigned kchunks = level_chunks(g);
+  const int kcc = run_levels((unsigned)(C / 64), g.nz + 1);  // one column a thread
   if (w.d6u) WD_TIMED(prof, KID_DIFF6, st, (launch_diff6(g, nl, s, w, st)));
   if (w.xkmh) WD_TIMED(prof, KID_SMAG, st, (launch_smag(g, nl, s, w, st)));
   if (w.ck_dz) WD_TIMED(prof, KID_CONSTK, st, (launch_constk(g, nl, s, w, st)));
@@ -2138,36 +2431,44 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
              (k_moist_factors<<<cell_grid(g), dim3(kFieldBx, kFieldBy), 0, st>>>(g, s, w)));
   WD_TIMED(prof, KID_RUV, st,
            (k_ruv<<<dim3(blocks_for(C, bs), kchunks), bs, 0, st>>>(g, s.u, s.v, s.mu_total, w.ru, w.rv)));
-  WD_TIMED(prof, KID_ROM, st, (k_rom<<<rom_blocks(g), 64, 0, st>>>(g, w.ru, w.rv, w.rom)));
+  const int bw = column_block_waves(g.nz);  // 0: too deep for the column-block kernels
+  if (bw > 0 && rom_blocks(g) <= kFewBlocks)
+    WD_TIMED(prof, KID_ROM, st,
+             (k_rom_block<<<rom_blocks(g), dim3(64, bw), (size_t)g.nz * 64 * sizeof(double), st>>>(g, w.ru, w.rv, w.rom)));
+  else
+    WD_TIMED(prof, KID_ROM, st, (k_rom<<<rom_blocks(g), 64, 0, st>>>(g, w.ru, w.rv, w.rom)));
   WD_TIMED(prof, KID_PREP_2D, st, (k_prep_2d<<<blocks_for(C, bs), bs, 0, st>>>(g, s, w, rk_step)));
   // k_prep_col writes the large-step diagnostics the tendency kernels read
-  WD_TIMED(prof, KID_PREP_COL, st, (k_prep_col<<<blocks_for(C, bs), bs, 0, st>>>(g, s, w)));
+  WD_TIMED(prof, KID_PREP_COL, st, (k_prep_col<<<dim3(blocks_for(C, bs), runs_of(g.nz + 1, kcc)), bs, 0, st>>>(g, s, w, kcc)));
   const size_t CU = (size_t)g.ny * (g.nx + 1), CV = (size_t)(g.ny + 1) * g.nx;
-  const unsigned tu_tiles = tend_u_tiles(g), tv_tiles = tend_v_tiles(g), tt_tiles = tend_t_tiles(g);
+  const int kcu = run_levels(tend_u_tiles(g) * kTendURows, g.nz), kcv = run_levels(tend_v_tiles(g) * kTendURows, g.nz),
+            kct = run_levels(tend_t_tiles(g) * kTendURows, g.nz);
+  const dim3 tu_tiles(tend_u_tiles(g), runs_of(g.nz, kcu)), tv_tiles(tend_v_tiles(g), runs_of(g.nz, kcv)),
+      tt_tiles(tend_t_tiles(g), runs_of(g.nz, kct)), tw_blocks(blocks_for(C, bs), runs_of(g.nz + 1, kcc));
   const dim3 tu_block(64, kTendURows);
   if (nl.mixed) {
-    WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<float, false><<<tu_tiles, tu_block, 0, st>>>(g, s, w)));
-    WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<float, false><<<tv_tiles, tu_block, 0, st>>>(g, s, w)));
-    WD_TIMED(prof, KID_TEND_W, st, (k_tend_w<float><<<blocks_for(C, bs), bs, 0, st>>>(g, s, w)));
+    WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<float, false><<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
+    WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<float, false><<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
+    WD_TIMED(prof, KID_TEND_W, st, (k_tend_w<float><<<tw_blocks, bs, 0, st>>>(g, s, w, kcc)));
     if (limit_theta)
       WD_TIMED(prof, KID_LIMITER, st, (launch_limiter<float>(g, nl, s, w, theta_lim, nl.scalar_adv_opt, st)));
     else
       WD_TIMED(prof, KID_TEND_T, st,
-               (k_tend_t<float><<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt)));
+               (k_tend_t<float><<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt, kct)));
   } else {
     if (w.cqu) {
-      WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<double, true><<<tu_tiles, tu_block, 0, st>>>(g, s, w)));
-      WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<double, true><<<tv_tiles, tu_block, 0, st>>>(g, s, w)));
+      WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<double, true><<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
+      WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<double, true><<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
     } else {
-      WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<double, false><<<tu_tiles, tu_block, 0, st>>>(g, s, w)));
-      WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<double, false><<<tv_tiles, tu_block, 0, st>>>(g, s, w)));
+      WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<double, false><<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
+      WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<double, false><<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
     }
-    WD_TIMED(prof, KID_TEND_W, st, (k_tend_w<double><<<blocks_for(C, bs), bs, 0, st>>>(g, s, w)));
+    WD_TIMED(prof, KID_TEND_W, st, (k_tend_w<double><<<tw_blocks, bs, 0, st>>>(g, s, w, kcc)));
     if (limit_theta)
       WD_TIMED(prof, KID_LIMITER, st, (launch_limiter<double>(g, nl, s, w, theta_lim, nl.scalar_adv_opt, st)));
     else
       WD_TIMED(prof, KID_TEND_T, st,
-               (k_tend_t<double><<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt)));
+               (k_tend_t<double><<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt, kct)));
   }
   // the species' coupled tendencies with the same transport velocities: the
   // plain h5/v3 advection, the limiter on the final stage from the step
@@ -2180,7 +2481,7 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
                                          nl.moist_adv_opt, st)));
       else
         WD_TIMED(prof, KID_MOIST, st,
-                 (k_tend_t<double><<<tt_tiles, tu_block, 0, st>>>(g, w, s.q[sp], 0.0, w.qt[sp], nullptr, nullptr)));
+                 (k_tend_t<double><<<tt_tiles, tu_block, 0, st>>>(g, w, s.q[sp], 0.0, w.qt[sp], nullptr, nullptr, kct)));
     }
   // the Coriolis force joins the coupled u/v tendencies after the PGF
   if (g.rot) {
@@ -2192,6 +2493,17 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
   WD_TIMED(prof, KID_PREP_FACES, st, (k_prep_faces<<<blocks_for(F, bs), bs, 0, st>>>(g, w)));
   WD_TIMED(prof, KID_PREP_U, st, (k_prep_u<<<dim3(blocks_for(CU, bs), kchunks), bs, 0, st>>>(g, s, w)));
   WD_TIMED(prof, KID_PREP_V, st, (k_prep_v<<<dim3(blocks_for(CV, bs), kchunks), bs, 0, st>>>(g, s, w)));
+  const unsigned row_tiles = (unsigned)((g.nx + kColOwned - 1) / kColOwned) * (unsigned)g.ny;
+  if (bw > 0 && row_tiles <= kFewBlocks) {
+    const dim3 block(64, bw);
+    if (nl.mixed)
+      WD_TIMED(prof, KID_COL_SETUP, st, (k_col_setup_block<float, false><<<row_tiles, block, 0, st>>>(g, nl, s, w, dts)));
+    else if (w.cqwr)
+      WD_TIMED(prof, KID_COL_SETUP, st, (k_col_setup_block<double, true><<<row_tiles, block, 0, st>>>(g, nl, s, w, dts)));
+    else
+      WD_TIMED(prof, KID_COL_SETUP, st, (k_col_setup_block<double, false><<<row_tiles, block, 0, st>>>(g, nl, s, w, dts)));
+    return hipGetLastError();
+  }
   const unsigned col_tiles = col_setup_tiles(g);
   const dim3 col_block(64, kColRows);
   if (nl.mixed) {
