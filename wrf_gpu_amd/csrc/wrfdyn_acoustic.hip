@@ -36,11 +36,11 @@ __device__ inline double dpn_ac(const DGrid& g, const double* __restrict__ p, in
 // levels k and k-1; the bottom and rigid-lid top faces use three levels).
 // ---------------------------------------------------------------------------
 // WET: the state carries moisture (cqu/cqv scale the pressure gradient); dry launches fold them to 1
-template <int BX, int BY, class TT, bool WET>
+template <int BX, int BY, class TT, bool WET, bool RUNS>
 __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState s, DWork w,
                                      double dts, int first, int kc) {
   const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
+  const int k0 = RUNS ? (int)B.y * kc : 0, k1 = RUNS && k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   // waves overlap by one lane: lanes 1..BX-1 own faces, lane 0 holds the
   // column west of the first owned face
   const unsigned nbx = (nx + 1 + BX - 2) / (BX - 1);
@@ -269,10 +269,10 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
   }
 }
 
-template <int BX, int BY, class TT, bool WET>
+template <int BX, int BY, class TT, bool WET, bool RUNS>
 __global__ void __launch_bounds__(BX * BY) k_uv(DGrid g, DState s, DWork w, double dts, int first, int kc) {
   __shared__ double sh[2][BY][7][BX];
-  b_uv<BX, BY, TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, dts, first, kc);
+  b_uv<BX, BY, TT, WET, RUNS>(hw_blk(), &sh[0][0][0][0], g, s, w, dts, first, kc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1299,6 +1299,7 @@ __device__ __forceinline__ void b_column_block(const unsigned tile, const int tx
   const double msfty = ldo(g.msfty, c8);
   const double eps_p = 1.0 + nl.epssm, eps_m = 1.0 - nl.epssm;
   const double mut = ldo(w.mut, c8), muts_old = ldo(w.muts, c8);
+  const double wsfc = c == 0 ? ldo(w.wsfc, c8) : 0.0;
   // levels are clamped for the loads, so that every load is in bounds
   auto mlev = [&](int k) { return k < 0 ? 0 : (k < nz ? k : nz - 1); };
   auto wlev = [&](int f) { return f < 0 ? 0 : (f <= nz ? f : nz); };
@@ -1542,7 +1543,7 @@ __device__ __forceinline__ void b_column_block(const unsigned tile, const int tx
                                    ((g.rdnw[f] * c2a[r]) / (mh * mf) + (g.rdnw[f - 1] * c2a_m) / (mh_m * mf));
         cal[r] = 1.0 / (b - ca[r] * cg[r]);
       } else {
-        wn[r] = f == 0 ? ldo(w.wsfc, c8) : 0.0;  // terrain surface w, rigid lid
+        wn[r] = f == 0 ? wsfc : 0.0;  // terrain surface w, rigid lid
       }
       ta_l = ta_u;
       bl = buoy[r];
@@ -1555,6 +1556,10 @@ __device__ __forceinline__ void b_column_block(const unsigned tile, const int tx
   phase_cut(f0);
 
   // ---- Thomas sweeps, the carried value from wave to wave ----
+  const bool damp = nl.damp_opt == 3 && nl.dampcoef > 0.0;
+  double ph1c[R], ph1_top, ph0;  // for the damping and the phi finish
+#pragma unroll
+  for (int r = 0; r < R; ++r) ph1c[r] = 0.0;
   {
     for (int q = 0; q < KT; ++q) {
       if (c == q) {
@@ -1568,6 +1573,13 @@ __device__ __forceinline__ void b_column_block(const unsigned tile, const int tx
       }
       __syncthreads();
     }
+    if (damp) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) ph1c[r] = ldo(w.ph1t, woff(f0 + r));
+    }
+    ph1_top = ldo(w.ph1t, woff(nz));
+    ph0 = ldo(w.ph_work, c8);
+    fence_sched();
     for (int q = KT - 1; q >= 0; --q) {
       if (c == q) {
         double next = q < KT - 1 ? carry[tx] : 0.0;
@@ -1587,8 +1599,7 @@ __device__ __forceinline__ void b_column_block(const unsigned tile, const int tx
   // ---- damping, the phi finish (rhs becomes the new ph work) ----
   {
     const double hdepth = nl.zdamp;
-    const double hbot = ldo(w.ph1t, woff(nz)) / kG - hdepth;
-    const bool damp = nl.damp_opt == 3 && nl.dampcoef > 0.0;
+    const double hbot = ph1_top / kG - hdepth;
     fence_sched();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -1596,10 +1607,10 @@ __device__ __forceinline__ void b_column_block(const unsigned tile, const int tx
       if (f > nz) continue;
       const unsigned q = c8 + (unsigned)f * plane;
       if (f == 0) {
-        rhs[r] = ldo(w.ph_work, c8);  // the surface ph work is unchanged
+        rhs[r] = ph0;  // the surface ph work is unchanged
       } else {
         if (damp) {
-          const double hk = ldo(w.ph1t, q) / kG;
+          const double hk = ph1c[r] / kG;
           if (hk >= hbot) {  // below the layer the weight is 0 and w passes through
             const double sn = wd_sin(((0.5 * kPi) * (hk - hbot)) / hdepth);
             const double dampwt = (dts * nl.dampcoef) * (sn * sn);
@@ -1675,7 +1686,7 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
   }
   struct Lv {
     double ww, wsave, phw, php, pht;           // w level f
-    double th, thw, ptot, ppert, pwork, pb;    // mass level f
+    double th, thw, pwork, pb;                 // mass level f
   };
   auto load = [&](int f, Lv& L) {
     const unsigned q = c8 + (unsigned)f * pl8;
@@ -1687,8 +1698,6 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
     if (f < nz) {
       L.th = ldo(s.theta, q);
       L.thw = ldo(w.th_work, q);
-      L.ptot = ldo(s.p_total, q);
-      L.ppert = ldo(s.p_pert, q);
       L.pwork = ldo(w.p, q);
       L.pb = ldo(w.pb, q);
     }
@@ -1729,7 +1738,7 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
       double theta_pert = (prev.thw + t_save * mch) / safe_den(msh);
       double theta = theta_pert + kT0;
       sto(s.theta, qk, theta);
-      double p_base = prev.ptot - prev.ppert;
+      double p_base = prev.pb;  // p_total - p' of the stage's state, as k_prep_col formed it
       double p_total = p_base + prev.pwork;
       double p_pert = prev.pwork;
       double muts_r = mub + mu_pert_new;
@@ -1867,11 +1876,11 @@ hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DS
   const int kc = run_levels(uv_tiles(g) * kUvBy, g.nz);
   const dim3 uvgrid(uv_tiles(g), runs_of(g.nz, kc));
   if (nl.mixed) {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, float, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
+    WD_TIMED(prof, KID_UV, st, (WD_RUNS(uvgrid.y, k_uv, BX, BY, float, false)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
   } else if (w.cqu) {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, true><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
+    WD_TIMED(prof, KID_UV, st, (WD_RUNS(uvgrid.y, k_uv, BX, BY, double, true)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
   } else {
-    WD_TIMED(prof, KID_UV, st, (k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
+    WD_TIMED(prof, KID_UV, st, (WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
   }
   // the LDS-tiled kernel has no moisture factor: a moist state runs the column march
   return launch_column_tile(w.cqwr ? kColumnMarch : column_tile, g, nl, s, w, dts, first, st, prof);
@@ -1886,7 +1895,7 @@ hipError_t launch_substep_part(int part, const DGrid& g, const DNamelist& nl, co
   if (part == 0) {
     const int kc = run_levels(uv_tiles(g) * kUvBy, g.nz);
     const dim3 uvgrid(uv_tiles(g), runs_of(g.nz, kc));
-    k_uv<BX, BY, double, false><<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc);
+    WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc);
   } else if (part == 1) {
     k_column_mu<double><<<column_mu_tiles(g), dim3(64, kMuRows), 0, st>>>(g, nl, s, w, dts, first);
   } else if (part == 2) {

@@ -125,7 +125,10 @@ int check_state(wd_handle* h, const wd_state* st, wd::DState* out, int moist_fla
 // refused during capture).
 int enqueue_steps(wd_handle* h, const wd::DState& ds, int n_large_steps, hipStream_t s) {
   const wd::DGrid& g = h->g;
-  const wd::DWork& w = h->w;
+  wd::DWork w = h->w;
+  // the column block forms a and alpha from gamma: k_col_setup stores them for
+  // the other column kernels only
+  if (h->column_tile == wd::kColumnMarch && wd::column_block_waves(g.nz) > 0) w.ca = w.calpha = nullptr;
   const size_t M = (size_t)g.nz * g.ny * g.nx, Wn = (size_t)(g.nz + 1) * g.ny * g.nx;
   const size_t U = (size_t)g.nz * g.ny * (g.nx + 1), V = (size_t)g.nz * (g.ny + 1) * g.nx;
   const size_t C = (size_t)g.ny * g.nx;

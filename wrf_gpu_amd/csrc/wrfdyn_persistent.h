@@ -114,7 +114,7 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       b_prep_faces(flat, M.g, M.w);
       break;
     case PK_PREP_COL:
-      b_prep_col(flat, M.g, M.s, M.w, (int)S.aux);
+      b_prep_col<false>(flat, M.g, M.s, M.w, 0);
       break;
     case PK_PREP_U:
       b_prep_u(flat, M.g, M.s, M.w);
@@ -123,16 +123,16 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       b_prep_v(flat, M.g, M.s, M.w);
       break;
     case PK_TEND_U:
-      b_tend_u<TT, false>(tile, lds, M.g, M.s, M.w, (int)S.aux);
+      b_tend_u<TT, false, false>(tile, lds, M.g, M.s, M.w, 0);
       break;
     case PK_TEND_V:
-      b_tend_v<TT, false>(tile, lds, M.g, M.s, M.w, (int)S.aux);
+      b_tend_v<TT, false, false>(tile, lds, M.g, M.s, M.w, 0);
       break;
     case PK_TEND_W:
-      b_tend_w<TT>(flat, M.g, M.s, M.w, (int)S.aux);
+      b_tend_w<TT, false>(flat, M.g, M.s, M.w, 0);
       break;
     case PK_TEND_T:
-      b_tend_t<TT>(tile, lds, M.g, M.w, M.s.theta, kT0, M.w.tht, M.w.d6t, M.w.smt, (int)S.aux);
+      b_tend_t<TT, false>(tile, lds, M.g, M.w, M.s.theta, kT0, M.w.tht, M.w.d6t, M.w.smt, 0);
       break;
     case PK_CORIOLIS:
       b_coriolis<TT>(flat, M.g, M.s, M.w, S.aux);
@@ -141,7 +141,7 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       b_col_setup<TT, false>(tile, lds, M.g, M.nl, M.s, M.w, S.dts);
       break;
     case PK_UV:
-      b_uv<kUvBx, kUvBy, TT, false>(tile, lds, M.g, M.s, M.w, S.dts, S.first, (int)S.aux);
+      b_uv<kUvBx, kUvBy, TT, false, false>(tile, lds, M.g, M.s, M.w, S.dts, S.first, 0);
       break;
     case PK_COLUMN_MU:
       b_column_mu<TT>(tile, lds, M.g, M.nl, M.s, M.w, S.dts, S.first);
@@ -346,16 +346,16 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
           case PK_ROM: S.gx = rom_blocks(g); break;
           case PK_PREP_2D: S.gx = blocks_for(C, 256); break;
           case PK_PREP_FACES: S.gx = blocks_for(CU + CV, 256); break;
-          case PK_PREP_COL: S.gx = blocks_for(C, 256); S.aux = (unsigned)(g.nz + 1); break;
+          case PK_PREP_COL: S.gx = blocks_for(C, 256); break;
           case PK_PREP_U: S.gx = blocks_for(CU, 256); S.gy = level_chunks(g); break;
           case PK_PREP_V: S.gx = blocks_for(CV, 256); S.gy = level_chunks(g); break;
-          case PK_TEND_U: S.gx = tend_u_tiles(g); S.aux = (unsigned)(g.nz); break;
-          case PK_TEND_V: S.gx = tend_v_tiles(g); S.aux = (unsigned)(g.nz); break;
-          case PK_TEND_W: S.gx = blocks_for(C, 256); S.aux = (unsigned)(g.nz + 1); break;
-          case PK_TEND_T: S.gx = tend_t_tiles(g); S.aux = (unsigned)(g.nz); break;
+          case PK_TEND_U: S.gx = tend_u_tiles(g); break;
+          case PK_TEND_V: S.gx = tend_v_tiles(g); break;
+          case PK_TEND_W: S.gx = blocks_for(C, 256); break;
+          case PK_TEND_T: S.gx = tend_t_tiles(g); break;
           case PK_CORIOLIS: S.gx = coriolis_blocks(g); S.aux = coriolis_u_blocks(g); break;
           case PK_COL_SETUP: S.gx = col_setup_tiles(g); break;
-          case PK_UV: S.gx = uv_tiles(g); S.aux = (unsigned)(g.nz); break;
+          case PK_UV: S.gx = uv_tiles(g); break;
           case PK_COLUMN_MU: S.gx = column_mu_tiles(g); break;
           case PK_COLUMN_W: S.gx = blocks_for(C, 256); break;
           case PK_FIN_UV: S.gx = blocks_for(CU + CV, 256); S.gy = fin_chunks(g); break;

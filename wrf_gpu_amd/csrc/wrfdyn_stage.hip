@@ -199,13 +199,13 @@ constexpr int kTendURows = 4;
 // come from the adjacent lanes (DPP), the rows j-3..j+3 inside the block and
 // rv at j+1 from the adjacent waves (LDS); the +-2, +-3 columns and rows
 // outside the block (or wrapping periodically) are loaded.
-template <class TT>
+template <class TT, bool RUNS>
 __device__ __forceinline__ void b_tend_t(const Blk& B, double* lds, DGrid g, DWork w,
                                          const double* __restrict__ th, double qoff, double* dst, const double* d6,
                                          const double* sm, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
+  const int k0 = RUNS ? (int)B.y * kc : 0, k1 = RUNS && k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   const unsigned nbx = (unsigned)(nx + 61) / 62;
   const unsigned tile = tile_id(g, B);
   const int tx = B.tx, ty = B.ty;
@@ -326,22 +326,22 @@ __device__ __forceinline__ void b_tend_t(const Blk& B, double* lds, DGrid g, DWo
   for (; k < k1; ++k) level(k);
 }
 
-template <class TT>
+template <class TT, bool RUNS>
 __global__ void __launch_bounds__(64 * kTendURows) k_tend_t(DGrid g, DWork w, const double* __restrict__ th,
                                                              double qoff, double* dst, const double* d6,
                                                              const double* sm, int kc) {
   __shared__ double sh[2][kTendURows][2][64];
-  b_tend_t<TT>(hw_blk(), &sh[0][0][0][0], g, w, th, qoff, dst, d6, sm, kc);
+  b_tend_t<TT, RUNS>(hw_blk(), &sh[0][0][0][0], g, w, th, qoff, dst, d6, sm, kc);
 }
 
 // advect_w_flux + _vertical_flux_div_w with a rigid lid
 // (flux_advection.py:1277-1329, 1410-1482) on w levels (nz+1, ny, nx); the
 // transport is _mass_to_full_levels of ru/rv (flux_advection.py:1332-1348).
-template <class TT>
+template <class TT, bool RUNS>
 __device__ __forceinline__ void b_tend_w(const Blk& B, DGrid g, DState s, DWork w, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const int f0 = (int)B.y * kc, f1 = f0 + kc < nz + 1 ? f0 + kc : nz + 1;  // this block's run of w levels
+  const int f0 = RUNS ? (int)B.y * kc : 0, f1 = RUNS && f0 + kc < nz + 1 ? f0 + kc : nz + 1;  // this block's run of w levels
   const size_t ncol = (size_t)ny * nx;
   const size_t c = (size_t)tile_id(g, B) * B.bdx + B.tx;
   if (c >= ncol) return;
@@ -489,20 +489,20 @@ __device__ __forceinline__ void b_tend_w(const Blk& B, DGrid g, DState s, DWork 
   for (; f < f1; ++f) level(f);
 }
 
-template <class TT>
+template <class TT, bool RUNS>
 __global__ void __launch_bounds__(256) k_tend_w(DGrid g, DState s, DWork w, int kc) {
-  b_tend_w<TT>(hw_blk(), g, s, w, kc);
+  b_tend_w<TT, RUNS>(hw_blk(), g, s, w, kc);
 }
 
 // advect_u_flux (flux_advection.py:1131-1202) + large_step_horizontal_pgf x
 // (rk_addtend_dry.py:329-343, 357-361) on u faces (nz, ny, nx+1).  Face nx
 // repeats face 0's advection (periodic); the PGF uses edge-padded pairs.
 // WET: the moisture factor cqu scales the PGF; dry launches fold it to 1.
-template <class TT, bool WET>
+template <class TT, bool WET, bool RUNS>
 __device__ __forceinline__ void b_tend_u(const Blk& B, double* lds, DGrid g, DState s, DWork w, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
+  const int k0 = RUNS ? (int)B.y * kc : 0, k1 = RUNS && k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   // Blocks of kTendURows rows of one 64-lane wave each; waves overlap by one
   // lane either side (lanes 1..62 own u faces).  Each lane loads its own face
   // (wrapped), its own mass column ia and the PGF's right column; the +-1
@@ -717,10 +717,10 @@ __device__ __forceinline__ void b_tend_u(const Blk& B, double* lds, DGrid g, DSt
   }
 }
 
-template <class TT, bool WET>
+template <class TT, bool WET, bool RUNS>
 __global__ void __launch_bounds__(64 * kTendURows) k_tend_u(DGrid g, DState s, DWork w, int kc) {
   __shared__ double sh[2][kTendURows][2][64];
-  b_tend_u<TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, kc);
+  b_tend_u<TT, WET, RUNS>(hw_blk(), &sh[0][0][0][0], g, s, w, kc);
 }
 
 // advect_v_flux (flux_advection.py:1205-1274) + large_step_horizontal_pgf y
@@ -730,11 +730,11 @@ __global__ void __launch_bounds__(64 * kTendURows) k_tend_u(DGrid g, DState s, D
 // k_tend_v's LDS fields: v, ru, rv, and the six PGF north-row values
 constexpr int kTendVFields = 9;
 
-template <class TT, bool WET>
+template <class TT, bool WET, bool RUNS>
 __device__ __forceinline__ void b_tend_v(const Blk& B, double* lds, DGrid g, DState s, DWork w, int kc) {
   constexpr bool MX = sizeof(TT) == sizeof(float);
   const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
+  const int k0 = RUNS ? (int)B.y * kc : 0, k1 = RUNS && k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   // Blocks of kTendURows v-face rows of one 64-lane wave each; waves overlap
   // by one lane either side (lanes 1..62 own columns).  Each lane loads its
   // own face (collapsed row ja, column wrapped), its own mass column and the
@@ -969,10 +969,10 @@ __device__ __forceinline__ void b_tend_v(const Blk& B, double* lds, DGrid g, DSt
   }
 }
 
-template <class TT, bool WET>
+template <class TT, bool WET, bool RUNS>
 __global__ void __launch_bounds__(64 * kTendURows) k_tend_v(DGrid g, DState s, DWork w, int kc) {
   __shared__ double sh[2][kTendURows][kTendVFields][64];
-  b_tend_v<TT, WET>(hw_blk(), &sh[0][0][0][0], g, s, w, kc);
+  b_tend_v<TT, WET, RUNS>(hw_blk(), &sh[0][0][0][0], g, s, w, kc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1113,6 +1113,7 @@ __global__ void __launch_bounds__(256) k_prep_v(DGrid g, DState s, DWork w) {
 //                c2a, php and calc_p_rho_wrf step 0 al, p
 //                (core/calc_p_rho.py:48-139)
 // ---------------------------------------------------------------------------
+template <bool RUNS>
 __device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWork w, int kc) {
   const size_t ncol = (size_t)g.ny * g.nx;
   const size_t c = (size_t)tile_id(g, B) * B.bdx + B.tx;
@@ -1143,7 +1144,7 @@ __device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWor
       L.th0 = ldo(w.th0, q);
     }
   };
-  const int f0 = (int)B.y * kc, f1 = f0 + kc < nz + 1 ? f0 + kc : nz + 1;  // this block's run of w levels
+  const int f0 = RUNS ? (int)B.y * kc : 0, f1 = RUNS && f0 + kc < nz + 1 ? f0 + kc : nz + 1;  // this block's run of w levels
   Lv cur{}, prev{};
   if (f0 > 0) load(f0 - 1, prev);
   load(f0, cur);
@@ -1221,8 +1222,9 @@ __device__ __forceinline__ void b_prep_col(const Blk& B, DGrid g, DState s, DWor
   }
 }
 
+template <bool RUNS>
 __global__ void __launch_bounds__(256) k_prep_col(DGrid g, DState s, DWork w, int kc) {
-  b_prep_col(hw_blk(), g, s, w, kc);
+  b_prep_col<RUNS>(hw_blk(), g, s, w, kc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1350,8 +1352,10 @@ __device__ __forceinline__ void b_col_setup(const Blk& B, double* lds, DGrid g, 
   if (owned) {
     sto(w.rw_tend, c8, 0.0 + ldt<TT>(w.wt, c8));
     stt<TT>(w.ph_tend, c8, 0.0);
-    sto(w.ca, c8, 0.0);
-    sto(w.calpha, c8, 1.0);
+    if (w.ca) {
+      sto(w.ca, c8, 0.0);
+      sto(w.calpha, c8, 1.0);
+    }
     sto(w.cgamma, c8, 0.0);
   }
   double gamma_prev = 0.0;
@@ -1440,8 +1444,10 @@ __device__ __forceinline__ void b_col_setup(const Blk& B, double* lds, DGrid g, 
       double al = 1.0 / (b - ak * gamma_prev);
       double gm = cc * al;
       if (owned) {
-        sto(w.ca, q, ak);
-        sto(w.calpha, q, al);
+        if (w.ca) {
+          sto(w.ca, q, ak);
+          sto(w.calpha, q, al);
+        }
         sto(w.cgamma, q, gm);
       }
       gamma_prev = gm;
@@ -1473,8 +1479,10 @@ __device__ __forceinline__ void b_col_setup(const Blk& B, double* lds, DGrid g, 
   double r2 = g.rdnw[nz - 1] * g.rdnw[nz - 1];
   double a_top = ((((-2.0 * cof) * r2) * c2a_m) * lid_flag) / top_denom_a;
   double b_top = 1.0 + (((2.0 * cof) * r2) * c2a_m) / top_denom_b;
-  sto(w.ca, qt, a_top);
-  sto(w.calpha, qt, 1.0 / (b_top - a_top * gamma_prev));
+  if (w.ca) {
+    sto(w.ca, qt, a_top);
+    sto(w.calpha, qt, 1.0 / (b_top - a_top * gamma_prev));
+  }
   sto(w.cgamma, qt, 0.0);
 }
 
@@ -1649,8 +1657,10 @@ __global__ void __launch_bounds__(1024) k_col_setup_block(DGrid g, DNamelist nl,
         gamma = f == 0 ? 0.0 : ck[r] * al;
         if (owned) {
           sto(w.cgamma, o, f < nz ? gamma : 0.0);
-          sto(w.ca, o, ak[r]);
-          sto(w.calpha, o, al);
+          if (w.ca) {
+            sto(w.ca, o, ak[r]);
+            sto(w.calpha, o, al);
+          }
         }
       }
       carry[tx] = gamma;
@@ -1682,9 +1692,21 @@ __global__ void __launch_bounds__(64 * kColRows) k_col_setup(DGrid g, DNamelist 
 // value once, and every stencil reads LDS.  One grid layer per level, so no
 // thread divides to find its point.
 constexpr int kFieldBx = 64, kFieldBy = 4, kTileRows = 16;
-inline dim3 tile_grid(int ncol, int nrow, int nlev) {
-  return dim3((unsigned)((ncol + kFieldBx - 1) / kFieldBx), (unsigned)((nrow + kTileRows - 1) / kTileRows),
-              (unsigned)nlev);
+// A level's tiles of kFieldBx columns x `rows` rows are one row of workgroups
+// (blockIdx.x), padded to a multiple of the 8 XCDs, blockIdx.z the level: an
+// XCD then runs the same contiguous band of rows at every level, and meets the
+// halo rows of its tiles and the planes of the levels below in its own L2.
+inline dim3 tile_grid(int ncol, int nrow, int nlev, int rows = kTileRows) {
+  const unsigned n = (unsigned)((ncol + kFieldBx - 1) / kFieldBx) * (unsigned)((nrow + rows - 1) / rows);
+  return dim3((n + kNumXcd - 1) / kNumXcd * kNumXcd, 1u, (unsigned)nlev);
+}
+// The corner of this workgroup's tile; false for the padding.
+__device__ inline bool tile_corner(int ncol, int nrow, int rows, int& i0, int& j0) {
+  const unsigned nbx = (unsigned)(ncol + kFieldBx - 1) / kFieldBx, nby = (unsigned)(nrow + rows - 1) / rows;
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  i0 = (int)(t % nbx) * kFieldBx;
+  j0 = (int)(t / nbx) * rows;
+  return t < nbx * nby;
 }
 // i wrapped into [0, n): the common in-range case without a division.
 __device__ inline int wrapc(int i, int n) {
@@ -1730,7 +1752,9 @@ __global__ void __launch_bounds__(256) k_diff6(DGrid g, const double* f, int kin
                                                const double* mu, double coef, double* out) {
   __shared__ double tile[kD6H][kD6W];
   const int tx = threadIdx.x, ty = threadIdx.y;
-  const int i0 = blockIdx.x * kFieldBx, j0 = blockIdx.y * kTileRows, k = blockIdx.z;
+  const int k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(ncol, nrow, kTileRows, i0, j0)) return;
   const double* lev = f + (size_t)k * nrow * ncol;
   for (int e = ty * kFieldBx + tx; e < kD6H * kD6W; e += kFieldBx * kFieldBy) {
     const int r = e / kD6W, c = e - r * kD6W;
@@ -1810,7 +1834,9 @@ __global__ void __launch_bounds__(256) k_constk(DGrid g, const double* f, int ki
                                                 const double* mu, double K, const double* dzp, double* out) {
   __shared__ double tf[kCkH][kCkW], tm[kCkH][kCkW];
   const int tx = threadIdx.x, ty = threadIdx.y;
-  const int i0 = blockIdx.x * kFieldBx, j0 = blockIdx.y * kTileRows, k = blockIdx.z;
+  const int k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(ncol, nrow, kTileRows, i0, j0)) return;
   const size_t P = (size_t)nrow * ncol;
   const double* lev = f + (size_t)k * P;
   for (int e = ty * kFieldBx + tx; e < kCkH * kCkW; e += kFieldBx * kFieldBy) {
@@ -1893,7 +1919,9 @@ __global__ void __launch_bounds__(256) k_smag_km(DGrid g, const double* u, const
   __shared__ double td12[kHdH][kHdW];  // D12 at the corners (q, c), q, c >= 1
   const int nx = g.nx, ny = g.ny;
   const int tx = threadIdx.x, ty = threadIdx.y;
-  const int i0 = blockIdx.x * kFieldBx, j0 = blockIdx.y * kTileRows, k = blockIdx.z;
+  const int k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(nx, ny, kTileRows, i0, j0)) return;
   for (int e = ty * kFieldBx + tx; e < kHdH * kHdW; e += kFieldBx * kFieldBy) {
     const int r = e / kHdW, c = e - r * kHdW;
     const int jj = wrapc(j0 - 1 + r, ny), ii = wrapc(i0 - 1 + c, nx);
@@ -1947,7 +1975,9 @@ __global__ void __launch_bounds__(256) k_hdiff(DGrid g, const double* f, int kin
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const int ncol = kind == 0 ? nx + 1 : nx, nrow = kind == 1 ? ny + 1 : ny;
   const int tx = threadIdx.x, ty = threadIdx.y;
-  const int i0 = blockIdx.x * kFieldBx, j0 = blockIdx.y * kTileRows, k = blockIdx.z;
+  const int k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(nx, ny, kTileRows, i0, j0)) return;
   const size_t plane = (size_t)ny * nx;
   const double* lev = f + (size_t)k * nrow * ncol;
   const double c1 = kind == 2 ? g.c1f[k] : g.c1h[k], c2 = kind == 2 ? g.c2f[k] : g.c2h[k];
@@ -2111,7 +2141,9 @@ struct LimFaces {
 // Each cell's minus faces (x face i, y face j, z face k; and face nz above
 // the top cell), computed once and stored.
 __global__ void __launch_bounds__(256) k_lim_faces(DGrid g, DState s, DWork w, LimScalar a, double dt) {
-  const int i = blockIdx.x * kFieldBx + threadIdx.x, j = blockIdx.y * kFieldBy + threadIdx.y, k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(g.nx, g.ny, kFieldBy, i0, j0)) return;
+  const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y, k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
   const double dxl = 1.0 / (1.0 / g.dx), dyl = 1.0 / (1.0 / g.dy);
   const size_t c = im(g, k, j, i);
@@ -2144,7 +2176,9 @@ __device__ inline LimFaces lim_faces(const DGrid& g, const DWork& w, int k, int 
 }
 
 __global__ void __launch_bounds__(256) k_lim_scale(DGrid g, DWork w, LimScalar a, int opt, double dt) {
-  const int i = blockIdx.x * kFieldBx + threadIdx.x, j = blockIdx.y * kFieldBy + threadIdx.y, k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(g.nx, g.ny, kFieldBy, i0, j0)) return;
+  const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y, k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const double rdx = 1.0 / g.dx, rdy = 1.0 / g.dy;
@@ -2198,7 +2232,9 @@ __device__ inline double lim_vface(int opt, double a, const double* sa, const do
 
 template <class TT>
 __global__ void __launch_bounds__(256) k_lim_tend(DGrid g, DWork w, LimScalar a, int opt) {
-  const int i = blockIdx.x * kFieldBx + threadIdx.x, j = blockIdx.y * kFieldBy + threadIdx.y, k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(g.nx, g.ny, kFieldBy, i0, j0)) return;
+  const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y, k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const double rdx = 1.0 / g.dx, rdy = 1.0 / g.dy;
@@ -2343,10 +2379,7 @@ void launch_coriolis(const DGrid& g, const DState& s, const DWork& w, hipStream_
   k_coriolis<TT><<<coriolis_blocks(g), 256, 0, st>>>(g, s, w, coriolis_u_blocks(g));
 }
 
-inline dim3 cell_grid(const DGrid& g) {
-  return dim3((unsigned)((g.nx + kFieldBx - 1) / kFieldBx), (unsigned)((g.ny + kFieldBy - 1) / kFieldBy),
-              (unsigned)g.nz);
-}
+inline dim3 cell_grid(const DGrid& g) { return tile_grid(g.nx, g.ny, g.nz, kFieldBy); }
 
 // One limited advection (opt 1 or 2) of the scalar `a`; the face and scale
 // arrays are shared, so limiter launches on one stream run one after another.
@@ -2376,7 +2409,9 @@ __device__ inline double qtot_at(const DState& s, size_t c) {
   return ((((s.q[0][c] + s.q[1][c]) + s.q[2][c]) + s.q[3][c]) + s.q[4][c]) + s.q[5][c];
 }
 __global__ void __launch_bounds__(256) k_moist_factors(DGrid g, DState s, DWork w) {
-  const int i = blockIdx.x * kFieldBx + threadIdx.x, j = blockIdx.y * kFieldBy + threadIdx.y, k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(g.nx, g.ny, kFieldBy, i0, j0)) return;
+  const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y, k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const double qc = qtot_at(s, im(g, k, j, i));
@@ -2395,7 +2430,9 @@ __global__ void __launch_bounds__(256) k_moist_factors(DGrid g, DState s, DWork 
 // column masses c1h mu + c2h of the step origin and of the finished stage,
 // every species of the cell in one thread.
 __global__ void __launch_bounds__(256) k_moist_update(DGrid g, DState s, DWork w, double dt_rk) {
-  const int i = blockIdx.x * kFieldBx + threadIdx.x, j = blockIdx.y * kFieldBy + threadIdx.y, k = blockIdx.z;
+  int i0, j0;
+  if (!tile_corner(g.nx, g.ny, kFieldBy, i0, j0)) return;
+  const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y, k = blockIdx.z;
   if (i >= g.nx || j >= g.ny) return;
   const size_t c2 = i2(g, j, i), c = im(g, k, j, i);
   const double mass_old = g.c1h[k] * w.mut0[c2] + g.c2h[k];
@@ -2419,6 +2456,7 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
   const size_t F = (size_t)g.ny * (g.nx + 1) + (size_t)(g.ny + 1) * g.nx;
   const unsigned kchunks = level_chunks(g);
   const int kcc = run_levels((unsigned)(C / 64), g.nz + 1);  // one column a thread
+  const dim3 pc_blocks(blocks_for(C, bs), runs_of(g.nz + 1, kcc));
   if (w.d6u) WD_TIMED(prof, KID_DIFF6, st, (launch_diff6(g, nl, s, w, st)));
   if (w.xkmh) WD_TIMED(prof, KID_SMAG, st, (launch_smag(g, nl, s, w, st)));
   if (w.ck_dz) WD_TIMED(prof, KID_CONSTK, st, (launch_constk(g, nl, s, w, st)));
@@ -2439,36 +2477,36 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
     WD_TIMED(prof, KID_ROM, st, (k_rom<<<rom_blocks(g), 64, 0, st>>>(g, w.ru, w.rv, w.rom)));
   WD_TIMED(prof, KID_PREP_2D, st, (k_prep_2d<<<blocks_for(C, bs), bs, 0, st>>>(g, s, w, rk_step)));
   // k_prep_col writes the large-step diagnostics the tendency kernels read
-  WD_TIMED(prof, KID_PREP_COL, st, (k_prep_col<<<dim3(blocks_for(C, bs), runs_of(g.nz + 1, kcc)), bs, 0, st>>>(g, s, w, kcc)));
+  WD_TIMED(prof, KID_PREP_COL, st, (WD_RUNS(pc_blocks.y, k_prep_col)<<<pc_blocks, bs, 0, st>>>(g, s, w, kcc)));
   const size_t CU = (size_t)g.ny * (g.nx + 1), CV = (size_t)(g.ny + 1) * g.nx;
   const int kcu = run_levels(tend_u_tiles(g) * kTendURows, g.nz), kcv = run_levels(tend_v_tiles(g) * kTendURows, g.nz),
             kct = run_levels(tend_t_tiles(g) * kTendURows, g.nz);
   const dim3 tu_tiles(tend_u_tiles(g), runs_of(g.nz, kcu)), tv_tiles(tend_v_tiles(g), runs_of(g.nz, kcv)),
-      tt_tiles(tend_t_tiles(g), runs_of(g.nz, kct)), tw_blocks(blocks_for(C, bs), runs_of(g.nz + 1, kcc));
+      tt_tiles(tend_t_tiles(g), runs_of(g.nz, kct)), tw_blocks = pc_blocks;
   const dim3 tu_block(64, kTendURows);
   if (nl.mixed) {
-    WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<float, false><<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
-    WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<float, false><<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
-    WD_TIMED(prof, KID_TEND_W, st, (k_tend_w<float><<<tw_blocks, bs, 0, st>>>(g, s, w, kcc)));
+    WD_TIMED(prof, KID_TEND_U, st, (WD_RUNS(tu_tiles.y, k_tend_u, float, false)<<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
+    WD_TIMED(prof, KID_TEND_V, st, (WD_RUNS(tv_tiles.y, k_tend_v, float, false)<<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
+    WD_TIMED(prof, KID_TEND_W, st, (WD_RUNS(tw_blocks.y, k_tend_w, float)<<<tw_blocks, bs, 0, st>>>(g, s, w, kcc)));
     if (limit_theta)
       WD_TIMED(prof, KID_LIMITER, st, (launch_limiter<float>(g, nl, s, w, theta_lim, nl.scalar_adv_opt, st)));
     else
       WD_TIMED(prof, KID_TEND_T, st,
-               (k_tend_t<float><<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt, kct)));
+               (WD_RUNS(tt_tiles.y, k_tend_t, float)<<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt, kct)));
   } else {
     if (w.cqu) {
-      WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<double, true><<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
-      WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<double, true><<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
+      WD_TIMED(prof, KID_TEND_U, st, (WD_RUNS(tu_tiles.y, k_tend_u, double, true)<<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
+      WD_TIMED(prof, KID_TEND_V, st, (WD_RUNS(tv_tiles.y, k_tend_v, double, true)<<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
     } else {
-      WD_TIMED(prof, KID_TEND_U, st, (k_tend_u<double, false><<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
-      WD_TIMED(prof, KID_TEND_V, st, (k_tend_v<double, false><<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
+      WD_TIMED(prof, KID_TEND_U, st, (WD_RUNS(tu_tiles.y, k_tend_u, double, false)<<<tu_tiles, tu_block, 0, st>>>(g, s, w, kcu)));
+      WD_TIMED(prof, KID_TEND_V, st, (WD_RUNS(tv_tiles.y, k_tend_v, double, false)<<<tv_tiles, tu_block, 0, st>>>(g, s, w, kcv)));
     }
-    WD_TIMED(prof, KID_TEND_W, st, (k_tend_w<double><<<tw_blocks, bs, 0, st>>>(g, s, w, kcc)));
+    WD_TIMED(prof, KID_TEND_W, st, (WD_RUNS(tw_blocks.y, k_tend_w, double)<<<tw_blocks, bs, 0, st>>>(g, s, w, kcc)));
     if (limit_theta)
       WD_TIMED(prof, KID_LIMITER, st, (launch_limiter<double>(g, nl, s, w, theta_lim, nl.scalar_adv_opt, st)));
     else
       WD_TIMED(prof, KID_TEND_T, st,
-               (k_tend_t<double><<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt, kct)));
+               (WD_RUNS(tt_tiles.y, k_tend_t, double)<<<tt_tiles, tu_block, 0, st>>>(g, w, s.theta, kT0, w.tht, w.d6t, w.smt, kct)));
   }
   // the species' coupled tendencies with the same transport velocities: the
   // plain h5/v3 advection, the limiter on the final stage from the step
@@ -2481,7 +2519,7 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
                                          nl.moist_adv_opt, st)));
       else
         WD_TIMED(prof, KID_MOIST, st,
-                 (k_tend_t<double><<<tt_tiles, tu_block, 0, st>>>(g, w, s.q[sp], 0.0, w.qt[sp], nullptr, nullptr, kct)));
+                 (WD_RUNS(tt_tiles.y, k_tend_t, double)<<<tt_tiles, tu_block, 0, st>>>(g, w, s.q[sp], 0.0, w.qt[sp], nullptr, nullptr, kct)));
     }
   // the Coriolis force joins the coupled u/v tendencies after the PGF
   if (g.rot) {
