@@ -774,7 +774,8 @@ __global__ void __launch_bounds__(TX * KT, (R <= 4 ? 3 : 1))
 }
 
 // ---------------------------------------------------------------------------
-// small_step_finish_wrf (core/small_step_finish.py:22-101)
+// small_step_finish_wrf (core/small_step_finish.py:22-101), from the stage's
+// state s into out (s itself, or other buffers)
 // ---------------------------------------------------------------------------
 __device__ inline double safe_den(double ms) { return fabs(ms) > 1.0e-12 ? ms : (ms >= 0.0 ? 1.0e-12 : -1.0e-12); }
 
@@ -783,7 +784,8 @@ __device__ inline double safe_den(double ms) { return fabs(ms) > 1.0e-12 ? ms : 
 constexpr int kFinChunk = 8;
 
 __device__ inline void fin_face_column(const DGrid& g, unsigned chunk, unsigned f, unsigned fplane8, double mus,
-                                       double mu, double msf, const double* __restrict__ xw, double* __restrict__ x) {
+                                       double mu, double msf, const double* __restrict__ xw, const double* x,
+                                       double* out) {
   const unsigned f8 = f * 8u;
   const int k0 = chunk * kFinChunk, k1 = k0 + kFinChunk < g.nz ? k0 + kFinChunk : g.nz;
 #pragma unroll 4
@@ -791,22 +793,22 @@ __device__ inline void fin_face_column(const DGrid& g, unsigned chunk, unsigned 
     const unsigned q = (unsigned)k * fplane8 + f8;
     const double ms = g.c1h[k] * mus + g.c2h[k];
     const double mc = g.c1h[k] * mu + g.c2h[k];
-    sto(x, q, (msf * ldo(xw, q) + ldo(x, q) * mc) / safe_den(ms));
+    sto(out, q, (msf * ldo(xw, q) + ldo(x, q) * mc) / safe_den(ms));
   }
 }
 
-__device__ __forceinline__ void b_fin_uv(const Blk& B, DGrid g, DState s, DWork w) {
+__device__ __forceinline__ void b_fin_uv(const Blk& B, DGrid g, DState s, DState out, DWork w) {
   const unsigned ncu = (unsigned)(g.ny * (g.nx + 1)), ncv = (unsigned)((g.ny + 1) * g.nx);
   const unsigned t = B.x * B.bdx + B.tx;
-  if (t < ncu) fin_face_column(g, B.y, t, ncu * 8u, w.muus[t], w.muu[t], g.msfuy[t], w.u_work, s.u);
+  if (t < ncu) fin_face_column(g, B.y, t, ncu * 8u, w.muus[t], w.muu[t], g.msfuy[t], w.u_work, s.u, out.u);
   else if (t < ncu + ncv) {
     const unsigned f = t - ncu;
-    fin_face_column(g, B.y, f, ncv * 8u, w.muvs[f], w.muv[f], g.msfvx[f], w.v_work, s.v);
+    fin_face_column(g, B.y, f, ncv * 8u, w.muvs[f], w.muv[f], g.msfvx[f], w.v_work, s.v, out.v);
   }
 }
 
-__global__ void __launch_bounds__(256) k_fin_uv(DGrid g, DState s, DWork w) {
-  b_fin_uv(hw_blk(), g, s, w);
+__global__ void __launch_bounds__(256) k_fin_uv(DGrid g, DState s, DState out, DWork w) {
+  b_fin_uv(hw_blk(), g, s, out, w);
 }
 
 // ---------------------------------------------------------------------------
@@ -1666,7 +1668,7 @@ __global__ void __launch_bounds__(1024) k_column_block(DGrid g, DNamelist nl, DS
 // several waves, each marching a run of kc levels (64x64x40: 53 -> 9 us).  The
 // state is updated in place, so a wave reads the old ph of the level below
 // its run before the workgroup's barrier, after which the runs are stored.
-__device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork w, int kc) {
+__device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DState out, DWork w, int kc) {
   const size_t ncol = (size_t)g.ny * g.nx;
   const size_t cb = (size_t)tile_id(g, B) * B.bdx + B.tx;
   const bool split = kc <= g.nz;
@@ -1681,8 +1683,8 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
   const bool hyps2 = g.hypsometric_opt == 2;
   if (f0 == 0 && cb < ncol) {
     double mu_base = s.mu_total[c] - s.mu_pert[c];
-    s.mu_pert[c] = mu_pert_new;
-    s.mu_total[c] = mu_base + mu_pert_new;
+    out.mu_pert[c] = mu_pert_new;
+    out.mu_total[c] = mu_base + mu_pert_new;
   }
   struct Lv {
     double ww, wsave, phw, php, pht;           // w level f
@@ -1723,12 +1725,12 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
     // w and ph at level f
     double ms = g.c1f[f] * muts + g.c2f[f];
     double mc = g.c1f[f] * mut + g.c2f[f];
-    sto(s.w, q, (msfty * cur.ww + cur.wsave * mc) / safe_den(ms));
+    sto(out.w, q, (msfty * cur.ww + cur.wsave * mc) / safe_den(ms));
     const double ph_pert = cur.phw + cur.php;
     const double ph_base = cur.pht - cur.php;
     const double ph_total = ph_base + ph_pert;
-    sto(s.ph_total, q, ph_total);
-    sto(s.ph_pert, q, ph_pert);
+    sto(out.ph_total, q, ph_total);
+    sto(out.ph_pert, q, ph_pert);
     if (f >= 1) {  // theta and p at mass level k = f - 1
       const int k = f - 1;
       const unsigned qk = q - pl8;
@@ -1737,7 +1739,7 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
       double t_save = prev.th - kT0;
       double theta_pert = (prev.thw + t_save * mch) / safe_den(msh);
       double theta = theta_pert + kT0;
-      sto(s.theta, qk, theta);
+      sto(out.theta, qk, theta);
       double p_base = prev.pb;  // p_total - p' of the stage's state, as k_prep_col formed it
       double p_total = p_base + prev.pwork;
       double p_pert = prev.pwork;
@@ -1764,8 +1766,8 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
       double ptot = p_from_theta_alt(theta, alt);
       double p_pert_new = ptot - prev.pb;
       double p_base2 = p_total - p_pert;
-      sto(s.p_total, qk, p_base2 + p_pert_new);
-      sto(s.p_pert, qk, p_pert_new);
+      sto(out.p_total, qk, p_base2 + p_pert_new);
+      sto(out.p_pert, qk, p_pert_new);
     }
     pht_prev = ph_total;
     php_prev = ph_pert;
@@ -1774,11 +1776,11 @@ __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DWork
   }
 }
 
-__global__ void __launch_bounds__(256) k_fin_col(DGrid g, DState s, DWork w) {
-  b_fin_col(hw_blk(), g, s, w, g.nz + 1);
+__global__ void __launch_bounds__(256) k_fin_col(DGrid g, DState s, DState out, DWork w) {
+  b_fin_col(hw_blk(), g, s, out, w, g.nz + 1);
 }
-__global__ void __launch_bounds__(1024) k_fin_col_runs(DGrid g, DState s, DWork w, int kc) {
-  b_fin_col(hw_blk(), g, s, w, kc);
+__global__ void __launch_bounds__(1024) k_fin_col_runs(DGrid g, DState s, DState out, DWork w, int kc) {
+  b_fin_col(hw_blk(), g, s, out, w, kc);
 }
 
 // Launch grids of the acoustic kernels, which the persistent ensemble step
@@ -1906,18 +1908,19 @@ hipError_t launch_substep_part(int part, const DGrid& g, const DNamelist& nl, co
   return hipGetLastError();
 }
 
-hipError_t launch_stage_finish(const DGrid& g, const DState& s, const DWork& w, hipStream_t st, Prof* prof) {
+hipError_t launch_stage_finish(const DGrid& g, const DState& s, const DState& out, const DWork& w, hipStream_t st,
+                               Prof* prof) {
   const unsigned bs = 256;
   const size_t UVcols = (size_t)g.ny * (g.nx + 1) + (size_t)(g.ny + 1) * g.nx;
   const size_t C = (size_t)g.ny * g.nx;
   const unsigned kchunks = fin_chunks(g);
-  WD_TIMED(prof, KID_FIN_UV, st, (k_fin_uv<<<dim3(blocks_for(UVcols, bs), kchunks), bs, 0, st>>>(g, s, w)));
+  WD_TIMED(prof, KID_FIN_UV, st, (k_fin_uv<<<dim3(blocks_for(UVcols, bs), kchunks), bs, 0, st>>>(g, s, out, w)));
   const int kc = column_wave_levels(g, g.nz + 1);
   if (kc <= g.nz) {
     const dim3 block(64, runs_of(g.nz + 1, kc));
-    WD_TIMED(prof, KID_FIN_COL, st, (k_fin_col_runs<<<blocks_for(C, 64), block, 0, st>>>(g, s, w, kc)));
+    WD_TIMED(prof, KID_FIN_COL, st, (k_fin_col_runs<<<blocks_for(C, 64), block, 0, st>>>(g, s, out, w, kc)));
   } else {
-    WD_TIMED(prof, KID_FIN_COL, st, (k_fin_col<<<blocks_for(C, bs), bs, 0, st>>>(g, s, w)));
+    WD_TIMED(prof, KID_FIN_COL, st, (k_fin_col<<<blocks_for(C, bs), bs, 0, st>>>(g, s, out, w)));
   }
   return hipGetLastError();
 }

@@ -269,7 +269,7 @@ hipError_t adjoint_large_step(const DGrid& g, const DNamelist& nl, const DWork& 
         ADJ_TRY(snap_carried(g, w, S, t, b++, it == 0 && part < 2, st));
       }
     }
-    ADJ_TRY(launch_stage_finish(g, S, w, st, nullptr));
+    ADJ_TRY(launch_stage_finish(g, S, S, w, st, nullptr));
   }
   // ---- reverse ----
   ADJ_TRY(hipMemsetAsync(t.bar[0], 0, (size_t)((char*)t.scr - (char*)t.bar[0]), st));  // every bar array

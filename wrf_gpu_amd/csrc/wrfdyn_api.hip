@@ -126,9 +126,37 @@ int check_state(wd_handle* h, const wd_state* st, wd::DState* out, int moist_fla
 int enqueue_steps(wd_handle* h, const wd::DState& ds, int n_large_steps, hipStream_t s) {
   const wd::DGrid& g = h->g;
   wd::DWork w = h->w;
-  // the column block forms a and alpha from gamma: k_col_setup stores them for
-  // the other column kernels only
-  if (h->column_tile == wd::kColumnMarch && wd::column_block_waves(g.nz) > 0) w.ca = w.calpha = nullptr;
+  // With the column block the stages pass the state on instead of advancing
+  // the caller's buffers three times, so the step origin is the caller's state
+  // itself and is not copied: stage 1 finishes into `mid`, stage 2 in place,
+  // stage 3 back into the caller's buffers.  mid is the origin copies' arrays
+  // and four that only the other column kernels use (a, alpha, the phi rhs and
+  // the forward-swept w; k_col_setup leaves a null a and alpha out).
+  const bool block = h->column_tile == wd::kColumnMarch && wd::column_block_waves(g.nz) > 0;
+  wd::DState mid = ds;
+  if (block) {
+    mid.u = w.u0;
+    mid.v = w.v0;
+    mid.w = w.w0;
+    mid.theta = w.th0;
+    mid.ph_pert = w.ph0;
+    mid.mu_pert = w.mu0;
+    mid.p_total = w.ca;
+    mid.p_pert = w.calpha;
+    mid.ph_total = w.wfwd;
+    mid.mu_total = w.rhs;
+    w.u0 = ds.u;
+    w.v0 = ds.v;
+    w.w0 = ds.w;
+    w.th0 = ds.theta;
+    w.ph0 = ds.ph_pert;
+    w.mu0 = ds.mu_pert;
+    for (int sp = 0; w.q0[0] && sp < wd::kNumMoist; ++sp) {
+      mid.q[sp] = w.q0[sp];
+      w.q0[sp] = ds.q[sp];
+    }
+    w.ca = w.calpha = w.wfwd = w.rhs = nullptr;
+  }
   const size_t M = (size_t)g.nz * g.ny * g.nx, Wn = (size_t)(g.nz + 1) * g.ny * g.nx;
   const size_t U = (size_t)g.nz * g.ny * (g.nx + 1), V = (size_t)g.nz * (g.ny + 1) * g.nx;
   const size_t C = (size_t)g.ny * g.nx;
@@ -151,7 +179,7 @@ int enqueue_steps(wd_handle* h, const wd::DState& ds, int n_large_steps, hipStre
         {w.u0, ds.u}, {w.v0, ds.v}, {w.w0, ds.w}, {w.th0, ds.theta}, {w.ph0, ds.ph_pert}, {w.mu0, ds.mu_pert}};
     const size_t sizes[] = {U, V, Wn, M, Wn, C};
     size_t tok = prof ? prof->begin(wd::KID_ORIGIN_COPY, s) : 0;
-    for (int q = 0; q < 6; ++q) {
+    for (int q = 0; q < 6 && !block; ++q) {
       e = hipMemcpyAsync(copies[q].first, copies[q].second, sizes[q] * sizeof(double), hipMemcpyDeviceToDevice, s);
       if (e != hipSuccess) return hip_fail(h, e, "hipMemcpyAsync(origin)");
     }
@@ -159,26 +187,28 @@ int enqueue_steps(wd_handle* h, const wd::DState& ds, int n_large_steps, hipStre
       e = hipMemcpyAsync(w.mut0, ds.mu_total, C * sizeof(double), hipMemcpyDeviceToDevice, s);
       if (e != hipSuccess) return hip_fail(h, e, "hipMemcpyAsync(origin)");
     }
-    if (w.q0[0])  // the species at the step origin (transport on)
+    if (w.q0[0] && !block)  // the species at the step origin (transport on)
       for (int sp = 0; sp < wd::kNumMoist; ++sp) {
         e = hipMemcpyAsync(w.q0[sp], ds.q[sp], M * sizeof(double), hipMemcpyDeviceToDevice, s);
         if (e != hipSuccess) return hip_fail(h, e, "hipMemcpyAsync(origin)");
       }
     if (prof) prof->end(tok, s);
     for (const StageDesc& sd : stages) {
-      e = wd::launch_stage_setup(g, h->nl, ds, w, sd.rk_step, sd.dts, s, prof);
+      const wd::DState& in = sd.rk_step == 1 ? ds : mid;
+      const wd::DState& out = sd.rk_step == 3 ? ds : mid;
+      e = wd::launch_stage_setup(g, h->nl, in, w, sd.rk_step, sd.dts, s, prof);
       if (e != hipSuccess) return hip_fail(h, e, "stage setup launch");
       for (int it = 0; it < sd.nsub; ++it) {
-        e = wd::launch_acoustic_substep(g, h->nl, ds, w, sd.dts, it == 0, h->column_tile, s, prof);
+        e = wd::launch_acoustic_substep(g, h->nl, in, w, sd.dts, it == 0, h->column_tile, s, prof);
         if (e != hipSuccess) return hip_fail(h, e, "acoustic substep launch");
       }
-      e = wd::launch_stage_finish(g, ds, w, s, prof);
+      e = wd::launch_stage_finish(g, in, out, w, s, prof);
       if (e != hipSuccess) return hip_fail(h, e, "stage finish launch");
       // the species' update with the stage's dt_rk: dt/3, dt/2, dt
       // (operational_mode.py:3527-3529)
       if (w.q0[0]) {
         const double dt_rk = sd.rk_step == 1 ? dt / 3.0 : (sd.rk_step == 2 ? 0.5 * dt : dt);
-        e = wd::launch_moist_update(g, ds, w, dt_rk, s, prof);
+        e = wd::launch_moist_update(g, out, w, dt_rk, s, prof);
         if (e != hipSuccess) return hip_fail(h, e, "moisture update launch");
       }
     }

@@ -216,10 +216,11 @@ inline int column_wave_levels(const DGrid& g, int n) {
 // wave: the waves a grid of nz levels needs, 0 where a workgroup's 16 are too
 // few.
 constexpr int kBlockLevels = 4;
-// The block forms of k_rom and k_col_setup pay while a launch has at most
-// kFewBlocks workgroups (two a CU): 64x64x40 (64 and 128 of them) 23 -> 6.5
-// and 58 -> 32 us, but at 433x433x50 49 -> 77 and 228 -> 613 us, since a
-// workgroup of one row shares no rows.
+// The block form of k_rom pays while a launch has at most kFewBlocks workgroups
+// (two a CU), that of k_col_setup, which needs more of a CU, up to half of
+// them: 64x64x40 (64 and 128 workgroups) 23 -> 6.5 and 58 -> 32 us,
+// 141x123x45 (369) 26 -> 11 and 70 -> 77 us, 433x433x50 (3031) 49 -> 77 and
+// 228 -> 613 us, since a workgroup of one row shares no rows.
 constexpr unsigned kFewBlocks = 512;
 inline int column_block_waves(int nz) { return nz + 1 <= 16 * kBlockLevels ? (nz + kBlockLevels) / kBlockLevels : 0; }
 inline unsigned runs_of(int n, int kc) { return (unsigned)((n + kc - 1) / kc); }

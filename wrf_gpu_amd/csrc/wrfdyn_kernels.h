@@ -126,8 +126,10 @@ hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DS
 hipError_t launch_moist_update(const DGrid& g, const DState& s, const DWork& w, double dt_rk, hipStream_t st,
                                Prof* prof);
 
-// small_step_finish + grid%p refresh.
-hipError_t launch_stage_finish(const DGrid& g, const DState& s, const DWork& w, hipStream_t st, Prof* prof);
+// small_step_finish + grid%p refresh, from the stage's state s into out (s
+// itself, or other buffers).
+hipError_t launch_stage_finish(const DGrid& g, const DState& s, const DState& out, const DWork& w, hipStream_t st,
+                               Prof* prof);
 
 // One kernel of a plain-FP64 acoustic substep with the column-march pair:
 // part 0 advance_uv (k_uv), 1 advance_mu_t + theta (k_column_mu), 2 advance_w

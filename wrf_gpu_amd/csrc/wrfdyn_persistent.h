@@ -135,7 +135,7 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       b_tend_t<TT, false>(tile, lds, M.g, M.w, M.s.theta, kT0, M.w.tht, M.w.d6t, M.w.smt, 0);
       break;
     case PK_CORIOLIS:
-      b_coriolis<TT>(flat, M.g, M.s, M.w, S.aux);
+      b_coriolis<TT>(flat, M.g, M.s, M.w, S.aux, M.g.nz);
       break;
     case PK_COL_SETUP:
       b_col_setup<TT, false>(tile, lds, M.g, M.nl, M.s, M.w, S.dts);
@@ -150,10 +150,10 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       b_column_w<TT>(flat, M.g, M.nl, M.s, M.w, S.dts, S.first);
       break;
     case PK_FIN_UV:
-      b_fin_uv(flat, M.g, M.s, M.w);
+      b_fin_uv(flat, M.g, M.s, M.s, M.w);
       break;
     case PK_FIN_COL:
-      b_fin_col(flat, M.g, M.s, M.w, M.g.nz + 1);
+      b_fin_col(flat, M.g, M.s, M.s, M.w, M.g.nz + 1);
       break;
     case PK_COLUMN_TILE:
       // FP64 only (the host never emits it for the mixed form); aux = levels per thread

@@ -2273,8 +2273,9 @@ __global__ void __launch_bounds__(256) k_lim_tend(DGrid g, DWork w, LimScalar a,
 // ---------------------------------------------------------------------------
 template <class TT>
 __device__ __forceinline__ void b_coriolis(const Blk& B, DGrid g, DState s, DWork w,
-                                           unsigned nbu) {
+                                           unsigned nbu, int kc) {
   const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int k0 = (int)B.y * kc, k1 = k0 + kc < nz ? k0 + kc : nz;  // this block's run of levels
   const size_t pl = (size_t)ny * nx, upl = (size_t)ny * (nx + 1), vpl = (size_t)(ny + 1) * nx;
   const bool ufaces = B.x < nbu;
   const size_t t = (size_t)(ufaces ? B.x : B.x - nbu) * B.bdx + B.tx;
@@ -2299,8 +2300,8 @@ __device__ __forceinline__ void b_coriolis(const Blk& B, DGrid g, DState s, DWor
       muv[q] = 0.5 * (s.mu_total[i2(g, clampi(jj - 1, 0, ny - 1), ii)] + s.mu_total[i2(g, clampi(jj, 0, ny - 1), ii)]);
       mvx[q] = g.msfvx[fv[q]];
     }
-    double rwl = rw_at(0, cl), rwr = rw_at(0, cr);
-    for (int k = 0; k < nz; ++k) {
+    double rwl = rw_at(k0, cl), rwr = rw_at(k0, cr);
+    for (int k = k0; k < k1; ++k) {
       double rv[4];
       for (int q = 0; q < 4; ++q) rv[q] = (s.v[(size_t)k * vpl + fv[q]] * (g.c1h[k] * muv[q] + g.c2h[k])) / mvx[q];
       const double rv_quad = 0.25 * (((rv[0] + rv[1]) + rv[2]) + rv[3]);
@@ -2330,8 +2331,8 @@ __device__ __forceinline__ void b_coriolis(const Blk& B, DGrid g, DState s, DWor
       muu[q] = 0.5 * (s.mu_total[i2(g, jj, clampi(ii - 1, 0, nx - 1))] + s.mu_total[i2(g, jj, clampi(ii, 0, nx - 1))]);
       muy[q] = g.msfuy[fu[q]];
     }
-    double rws = rw_at(0, cs), rwn = rw_at(0, cn);
-    for (int k = 0; k < nz; ++k) {
+    double rws = rw_at(k0, cs), rwn = rw_at(k0, cn);
+    for (int k = k0; k < k1; ++k) {
       double ru[4];
       for (int q = 0; q < 4; ++q) ru[q] = (s.u[(size_t)k * upl + fu[q]] * (g.c1h[k] * muu[q] + g.c2h[k])) / muy[q];
       const double ru_quad = 0.25 * (((ru[0] + ru[1]) + ru[2]) + ru[3]);
@@ -2348,8 +2349,8 @@ __device__ __forceinline__ void b_coriolis(const Blk& B, DGrid g, DState s, DWor
 }
 
 template <class TT>
-__global__ void __launch_bounds__(256) k_coriolis(DGrid g, DState s, DWork w, unsigned nbu) {
-  b_coriolis<TT>(hw_blk(), g, s, w, nbu);
+__global__ void __launch_bounds__(256) k_coriolis(DGrid g, DState s, DWork w, unsigned nbu, int kc) {
+  b_coriolis<TT>(hw_blk(), g, s, w, nbu, kc);
 }
 
 // Launch grids of the stage kernels, which the persistent ensemble step
@@ -2376,7 +2377,8 @@ inline unsigned coriolis_blocks(const DGrid& g) {
 
 template <class TT>
 void launch_coriolis(const DGrid& g, const DState& s, const DWork& w, hipStream_t st) {
-  k_coriolis<TT><<<coriolis_blocks(g), 256, 0, st>>>(g, s, w, coriolis_u_blocks(g));
+  const int kc = run_levels(coriolis_blocks(g) * 4u, g.nz);
+  k_coriolis<TT><<<dim3(coriolis_blocks(g), runs_of(g.nz, kc)), 256, 0, st>>>(g, s, w, coriolis_u_blocks(g), kc);
 }
 
 inline dim3 cell_grid(const DGrid& g) { return tile_grid(g.nx, g.ny, g.nz, kFieldBy); }
@@ -2532,7 +2534,7 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
   WD_TIMED(prof, KID_PREP_U, st, (k_prep_u<<<dim3(blocks_for(CU, bs), kchunks), bs, 0, st>>>(g, s, w)));
   WD_TIMED(prof, KID_PREP_V, st, (k_prep_v<<<dim3(blocks_for(CV, bs), kchunks), bs, 0, st>>>(g, s, w)));
   const unsigned row_tiles = (unsigned)((g.nx + kColOwned - 1) / kColOwned) * (unsigned)g.ny;
-  if (bw > 0 && row_tiles <= kFewBlocks) {
+  if (bw > 0 && row_tiles <= kFewBlocks / 2) {
     const dim3 block(64, bw);
     if (nl.mixed)
       WD_TIMED(prof, KID_COL_SETUP, st, (k_col_setup_block<float, false><<<row_tiles, block, 0, st>>>(g, nl, s, w, dts)));
