@@ -959,11 +959,11 @@ int wd_batch_create_persistent(wd_handle* const* members, const wd_state* states
   std::string why;
   if (!wd::persistent_program(pm, tiles, &segs, &phases, &why)) return fail(nullptr, WD_EINVAL, why);
   const bool mixed = pm[0].nl.mixed != 0;
-  const bool tile = std::any_of(column_kernel.begin(), column_kernel.end(), [](int k) { return k >= 0; });
+  const wd::PForm form = wd::persistent_form(segs);
   // as many workgroups as the GPU holds at once (the grid barrier needs every
   // one resident), a multiple of the 8 XCDs,
   int per_cu = 0, cus = 0;
-  e = wd::persistent_blocks_per_cu(mixed, tile, &per_cu);
+  e = wd::persistent_blocks_per_cu(mixed, form, &per_cu);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e != hipSuccess) return hip_fail(nullptr, e, "occupancy of the persistent step");
   // and no more than the largest phase has virtual blocks: fewer workgroups
@@ -1015,7 +1015,7 @@ int wd_batch_create_persistent(wd_handle* const* members, const wd_state* states
     wd_batch_destroy(b);
     return hip_fail(nullptr, e, "hipStreamBeginCapture");
   }
-  e = wd::launch_persistent_step(mixed, tile, grid, reinterpret_cast<const wd::PMember*>(base + o_mem),
+  e = wd::launch_persistent_step(mixed, form, grid, reinterpret_cast<const wd::PMember*>(base + o_mem),
                                  reinterpret_cast<const wd::PSeg*>(base + o_seg),
                                  reinterpret_cast<const wd::PPhase*>(base + o_ph), (int)phases.size(), b->bar, s0);
   hipGraph_t graph = nullptr;

@@ -181,11 +181,13 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
 // Levels per thread with which the persistent step runs a member's column
 // tile, 0 where it runs the column march.
 int persistent_column_levels(const DGrid& g, const DNamelist& nl, int column_tile);
-// Workgroups of the persistent kernel one CU holds at once.  `tile`: the
-// FP64 kernel that also carries the column tile, for a program with a
-// PK_COLUMN_TILE segment.
-hipError_t persistent_blocks_per_cu(bool mixed, bool tile, int* out);
-hipError_t launch_persistent_step(bool mixed, bool tile, unsigned grid, const PMember* members, const PSeg* segs,
+// The persistent kernel a program runs: with the column march, with the column
+// tile beside it (FP64), or with the column block (a small ensemble).
+enum class PForm { march, tile, block };
+PForm persistent_form(const std::vector<PSeg>& segs);
+// Workgroups of that kernel one CU holds at once.
+hipError_t persistent_blocks_per_cu(bool mixed, PForm form, int* out);
+hipError_t launch_persistent_step(bool mixed, PForm form, unsigned grid, const PMember* members, const PSeg* segs,
                                   const PPhase* phases, int n_phases, PBarrier* bar, hipStream_t st);
 
 // Adjoint of one plain-FP64 large step (wrfdyn_adjoint.hip).  The tape is

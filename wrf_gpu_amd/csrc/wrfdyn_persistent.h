@@ -42,6 +42,7 @@ enum PKind : int {
   PK_FIN_UV,
   PK_FIN_COL,
   PK_COLUMN_TILE,
+  PK_COLUMN_BLOCK,
 };
 
 namespace {
@@ -57,7 +58,13 @@ constexpr int kPersistTileLds = (6 * kPersistTileKt * kPersistTileLevels + 3) * 
 // The tile bodies share one LDS buffer, the size of the largest (k_tend_v's);
 // the kernel that also carries the column tile sizes it for that tile's
 // deepest grid.
+// The column block runs with kPersistBlockLevels levels a wave on the
+// workgroup's four waves.
+constexpr int kPersistBlockLevels = 13, kPersistBlockWaves = 4;
+constexpr int kPersistBlockNz = kPersistBlockLevels * kPersistBlockWaves - 1;
 constexpr int kPersistLds = 2 * kTendURows * kTendVFields * 64;
+constexpr int kPersistLdsBlock = std::max(kPersistLds, 2 * kPersistBlockNz * 64 + 64);
+static_assert(kBlockExch * kPersistBlockWaves <= kPersistBlockNz, "the exchanges fit the sums' plane");
 constexpr int kPersistLdsTile = std::max(kPersistLds, kPersistTileLds);
 static_assert(kPersistTileTx * kPersistTileKt == 256, "the column tile runs on a 256-thread workgroup");
 static_assert(2 * kTendURows * 2 * 64 <= kPersistLds, "k_tend_u / k_tend_t tile");
@@ -87,7 +94,7 @@ __device__ inline void origin_copy(const PMember& M, size_t e) {
 
 // Virtual block `local` of segment S, on the thread `tid` of a 256-thread
 // workgroup.
-template <bool MX, bool TILE>
+template <bool MX, PForm FORM>
 __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, unsigned local, unsigned tid,
                                             double* lds) {
   using TT = typename std::conditional<MX, float, double>::type;
@@ -155,9 +162,15 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
     case PK_FIN_COL:
       b_fin_col(flat, M.g, M.s, M.s, M.w, M.g.nz + 1);
       break;
+    case PK_COLUMN_BLOCK:
+      if constexpr (FORM == PForm::block)
+        b_column_block<kPersistBlockLevels, TT, false>(tile_id(M.g, flat), (int)(tid & 63u),
+                                                       __builtin_amdgcn_readfirstlane((int)(tid >> 6)),
+                                                       kPersistBlockWaves, lds, M.g, M.nl, M.s, M.w, S.dts, S.first);
+      break;
     case PK_COLUMN_TILE:
       // FP64 only (the host never emits it for the mixed form); aux = levels per thread
-      if constexpr (!MX && TILE) {
+      if constexpr (!MX && FORM == PForm::tile) {
         constexpr int TX = kPersistTileTx, KT = kPersistTileKt;
         const int tx = (int)(tid % TX), kt = (int)(tid / TX);
         const unsigned t = tile_id(M.g, flat);
@@ -174,6 +187,13 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       break;
   }
 }
+
+// Column blocks of all members up to which the step runs them: two for each of
+// the 256 workgroups that fit with them (one a CU).  One 64x64x40 member (128
+// of them) takes 2.30 ms a step with the block and 3.36 ms with the march, whose
+// 64 waves leave the GPU idle; larger ensembles fill it and keep the march's
+// two workgroups a CU.
+constexpr unsigned long long kPersistBlockTiles = 512;
 
 // s_waitcnt vmcnt(0) in the gfx9 encoding (vmcnt 0, expcnt 7, lgkmcnt 15):
 // every vector memory access the wave issued, stores included, has completed.
@@ -220,7 +240,7 @@ __device__ bool grid_barrier(PBarrier* bar, int* ok) {
 
 // One large step: the phases in order, the workgroup taking every
 // gridDim.x-th virtual block of each, with a grid barrier between phases.
-template <bool MX, bool TILE>
+template <bool MX, PForm FORM>
 __device__ __forceinline__ void step_phases(const PMember* __restrict__ members, const PSeg* __restrict__ segs,
                                             const PPhase* __restrict__ phases, int n_phases, PBarrier* bar,
                                             double* lds, int* ok) {
@@ -243,7 +263,7 @@ __device__ __forceinline__ void step_phases(const PMember* __restrict__ members,
       const unsigned local = v - S.vb0;
       if (local >= S.nvb) continue;  // the padding that aligns the next segment
       __syncthreads();               // the previous body's LDS reads are done
-      run_segment<MX, TILE>(S, members[S.member], local, tid, lds);
+      run_segment<MX, FORM>(S, members[S.member], local, tid, lds);
     }
     if (p + 1 < n_phases && !grid_barrier(bar, ok)) return;
   }
@@ -257,7 +277,7 @@ __global__ void __launch_bounds__(256) k_step_persistent(const PMember* __restri
                                                         PBarrier* bar) {
   __shared__ double lds[kPersistLds];
   __shared__ int ok;
-  step_phases<MX, false>(members, segs, phases, n_phases, bar, lds, &ok);
+  step_phases<MX, PForm::march>(members, segs, phases, n_phases, bar, lds, &ok);
 }
 
 // The FP64 step with the 16 x 16 column tile among its bodies, held to two
@@ -269,7 +289,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
                            const PPhase* __restrict__ phases, int n_phases, PBarrier* bar) {
   __shared__ double lds[kPersistLdsTile];
   __shared__ int ok;
-  step_phases<false, true>(members, segs, phases, n_phases, bar, lds, &ok);
+  step_phases<false, PForm::tile>(members, segs, phases, n_phases, bar, lds, &ok);
+}
+
+// The step of a small ensemble, whose members run the column block: it takes
+// more than half the register file, one workgroup a CU, which is what such an
+// ensemble fills.
+template <bool MX>
+__global__ void __launch_bounds__(256) k_step_persistent_block(const PMember* __restrict__ members,
+                                                               const PSeg* __restrict__ segs,
+                                                               const PPhase* __restrict__ phases, int n_phases,
+                                                               PBarrier* bar) {
+  __shared__ double lds[kPersistLdsBlock];
+  __shared__ int ok;
+  step_phases<MX, PForm::block>(members, segs, phases, n_phases, bar, lds, &ok);
 }
 
 }  // namespace
@@ -292,7 +325,15 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
   // levels per thread of the member's LDS column tile, 0 for the column march
   std::vector<int> tile_levels(nm);
   for (int m = 0; m < nm; ++m) tile_levels[m] = persistent_column_levels(members[m].g, members[m].nl, column_tiles[m]);
-  const bool any_march = std::count(tile_levels.begin(), tile_levels.end(), 0) > 0;
+  const bool any_tile = std::count(tile_levels.begin(), tile_levels.end(), 0) < nm;
+  // the column block instead of the march, where the launch is short of waves
+  std::vector<char> use_block(nm, 0);
+  unsigned long long block_tiles = 0;
+  for (const PMember& m : members) block_tiles += column_block_tiles(m.g);
+  for (int m = 0; m < nm; ++m)
+    use_block[m] = !any_tile && block_tiles <= kPersistBlockTiles && members[m].g.nz <= kPersistBlockNz;
+  bool any_march = false;
+  for (int m = 0; m < nm; ++m) any_march = any_march || (tile_levels[m] == 0 && !use_block[m]);
   const DNamelist& n0 = members[0].nl;
   for (int m = 0; m < nm; ++m) {
     const DNamelist& nl = members[m].nl;
@@ -327,7 +368,9 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
         const DNamelist& nl = members[m].nl;
         if (jb.kind == PK_CORIOLIS && !g.rot) continue;
         const bool march_kind = jb.kind == PK_COLUMN_MU || jb.kind == PK_COLUMN_W;
-        if ((march_kind && tile_levels[m] > 0) || (jb.kind == PK_COLUMN_TILE && tile_levels[m] == 0)) continue;
+        if ((march_kind && (tile_levels[m] > 0 || use_block[m])) || (jb.kind == PK_COLUMN_TILE && tile_levels[m] == 0) ||
+            (jb.kind == PK_COLUMN_BLOCK && !use_block[m]))
+          continue;
         const size_t C = (size_t)g.ny * g.nx, CU = (size_t)g.ny * (g.nx + 1), CV = (size_t)(g.ny + 1) * g.nx;
         PSeg S{};
         S.kind = jb.kind;
@@ -360,6 +403,7 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
           case PK_COLUMN_W: S.gx = blocks_for(C, 256); break;
           case PK_FIN_UV: S.gx = blocks_for(CU + CV, 256); S.gy = fin_chunks(g); break;
           case PK_FIN_COL: S.gx = blocks_for(C, 256); break;
+          case PK_COLUMN_BLOCK: S.gx = column_block_tiles(g); break;
           case PK_COLUMN_TILE:
             S.gx = (unsigned)((g.nx + kPersistTileTx - 1) / kPersistTileTx) * (unsigned)g.ny;
             S.aux = (unsigned)tile_levels[m];
@@ -395,7 +439,7 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
       const int first = it == 0 ? 1 : 0;
       add_phase({{PK_UV, rk, first}});
       // a member runs either the column-march pair or the LDS column tile
-      add_phase({{PK_COLUMN_MU, rk, first}, {PK_COLUMN_TILE, rk, first}});
+      add_phase({{PK_COLUMN_MU, rk, first}, {PK_COLUMN_BLOCK, rk, first}, {PK_COLUMN_TILE, rk, first}});
       if (any_march) add_phase({{PK_COLUMN_W, rk, first}});
     }
     add_phase({{PK_FIN_UV, rk, 0}, {PK_FIN_COL, rk, 0}});
@@ -403,24 +447,38 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
   return true;
 }
 
-hipError_t persistent_blocks_per_cu(bool mixed, bool tile, int* out) {
-  if (tile)
-    return mixed ? hipErrorInvalidValue
-                 : hipOccupancyMaxActiveBlocksPerMultiprocessor(out, k_step_persistent_tile, 256, 0);
-  return mixed ? hipOccupancyMaxActiveBlocksPerMultiprocessor(out, k_step_persistent<true>, 256, 0)
-               : hipOccupancyMaxActiveBlocksPerMultiprocessor(out, k_step_persistent<false>, 256, 0);
+PForm persistent_form(const std::vector<PSeg>& segs) {
+  for (const PSeg& S : segs) {
+    if (S.kind == PK_COLUMN_TILE) return PForm::tile;
+    if (S.kind == PK_COLUMN_BLOCK) return PForm::block;
+  }
+  return PForm::march;
 }
 
-hipError_t launch_persistent_step(bool mixed, bool tile, unsigned grid, const PMember* members, const PSeg* segs,
-                                  const PPhase* phases, int n_phases, PBarrier* bar, hipStream_t st) {
-  if (tile) {
-    if (mixed) return hipErrorInvalidValue;
-    k_step_persistent_tile<<<grid, 256, 0, st>>>(members, segs, phases, n_phases, bar);
-  } else if (mixed) {
-    k_step_persistent<true><<<grid, 256, 0, st>>>(members, segs, phases, n_phases, bar);
-  } else {
-    k_step_persistent<false><<<grid, 256, 0, st>>>(members, segs, phases, n_phases, bar);
+namespace {
+
+using PersistentKernel = void (*)(const PMember*, const PSeg*, const PPhase*, int, PBarrier*);
+
+PersistentKernel persistent_kernel(bool mixed, PForm form) {
+  switch (form) {
+    case PForm::tile: return mixed ? nullptr : k_step_persistent_tile;
+    case PForm::block: return mixed ? k_step_persistent_block<true> : k_step_persistent_block<false>;
+    default: return mixed ? k_step_persistent<true> : k_step_persistent<false>;
   }
+}
+
+}  // namespace
+
+hipError_t persistent_blocks_per_cu(bool mixed, PForm form, int* out) {
+  const PersistentKernel k = persistent_kernel(mixed, form);
+  return k ? hipOccupancyMaxActiveBlocksPerMultiprocessor(out, k, 256, 0) : hipErrorInvalidValue;
+}
+
+hipError_t launch_persistent_step(bool mixed, PForm form, unsigned grid, const PMember* members, const PSeg* segs,
+                                  const PPhase* phases, int n_phases, PBarrier* bar, hipStream_t st) {
+  const PersistentKernel k = persistent_kernel(mixed, form);
+  if (!k) return hipErrorInvalidValue;
+  k<<<grid, 256, 0, st>>>(members, segs, phases, n_phases, bar);
   return hipGetLastError();
 }
 
