@@ -36,7 +36,10 @@ __device__ inline double dpn_ac(const DGrid& g, const double* __restrict__ p, in
 // levels k and k-1; the bottom and rigid-lid top faces use three levels).
 // ---------------------------------------------------------------------------
 // WET: the state carries moisture (cqu/cqv scale the pressure gradient); dry launches fold them to 1
-template <int BX, int BY, class TT, bool WET, bool RUNS>
+// PREP: a stage's first substep, which forms the coupled work velocities of
+// small_step_prep from the step origin's and the stage's u and v, four reads,
+// instead of having k_prep_u/v write them and reading them back, eight passes
+template <int BX, int BY, class TT, bool WET, bool PREP, bool RUNS>
 __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState s, DWork w,
                                      double dts, int first, int kc) {
   const int nx = g.nx, ny = g.ny, nz = g.nz;
@@ -62,6 +65,7 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
   const size_t cs = i2(g, js, ic);  // v pair: (south, centre) on column ic == i
   double msf_u = 0.0, mudf_u = 0.0, muwsum_u = 0.0, muu = 0.0;
   double msf_v = 0.0, mudf_v = 0.0, muwsum_v = 0.0, muv = 0.0;
+  double muus = 0.0, msfuy = 1.0, muvs = 0.0, msfvx = 1.0;  // PREP
   if (do_u) {
     msf_u = g.msfux[i2u(g, j, i)] / g.msfuy[i2u(g, j, i)];
     double muw_l = w.muts[cw] - w.mut[cw];
@@ -69,6 +73,10 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     muwsum_u = muw_l + muw_r;
     mudf_u = ((-kEmdiv * g.dx) * (s.mudf[cc] - s.mudf[cw])) / g.msfuy[i2u(g, j, i)];
     muu = w.muu[i2u(g, j, i)];
+    if constexpr (PREP) {
+      muus = w.muus[i2u(g, j, i)];
+      msfuy = g.msfuy[i2u(g, j, i)];
+    }
   }
   if (do_v) {
     msf_v = g.msfvy[i2v(g, j, i)] / g.msfvx[i2v(g, j, i)];
@@ -78,6 +86,10 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     double msfvx_inv = 1.0 / g.msfvx[i2v(g, j, i)];
     mudf_v = ((-kEmdiv * g.dy) * (s.mudf[cc] - s.mudf[cs])) * msfvx_inv;
     muv = w.muv[i2v(g, j, i)];
+    if constexpr (PREP) {
+      muvs = w.muvs[i2v(g, j, i)];
+      msfvx = g.msfvx[i2v(g, j, i)];
+    }
   }
   // The inverse-density perturbation of the last calc_p_rho (core/calc_p_rho.py:
   // 48-183) is one divide from the new ph work, alt and the column mass, so it
@@ -140,7 +152,11 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     L.pc = ldo(P, ok + cc8);
     if (do_u) {
       const unsigned q = uq8 + (unsigned)k * upl8;
-      L.uw = ldo(w.u_work, q);
+      if constexpr (PREP) {
+        L.uw = ldo(w.u0, q);
+      } else {
+        L.uw = ldo(w.u_work, q);
+      }
       L.ut = ldt<TT>(w.ut, q);
     }
     if (do_v) {
@@ -152,7 +168,11 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
         L.phps = ldo(w.php, ok + cs8);
         L.ps = ldo(P, ok + cs8);
       }
-      L.vw = ldo(w.v_work, q);
+      if constexpr (PREP) {
+        L.vw = ldo(w.v0, q);
+      } else {
+        L.vw = ldo(w.v_work, q);
+      }
       L.vt = ldt<TT>(w.vt, q);
     }
     if (k + 2 < nz) {
@@ -201,6 +221,11 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
   Lv cur{};
   load(k0, cur);
   for (int k = k0; k < k1; ++k) {
+    double uo = 0.0, vo = 0.0;  // PREP: the stage's u and v (uw, vw: the origin's)
+    if constexpr (PREP) {
+      if (do_u) uo = ldo(s.u, uq8 + (unsigned)k * upl8);
+      if (do_v) vo = ldo(s.v, vq8 + (unsigned)k * vpl8);
+    }
     Lv nxt{};
     if (k + 1 < k1) load(k + 1, nxt);
     cur.alc = al_at(k, cur.altc, muts_c, muw_c, phc, cur.phc1);
@@ -222,8 +247,9 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     if (do_u) {
       const double phw1 = cur.phw1;
       const unsigned q = uq8 + (unsigned)k * upl8;
-      double u = cur.uw + dts * cur.ut;
       double mass_x = g.c1h[k] * muu + g.c2h[k];
+      const double uw0 = PREP ? ((g.c1h[k] * muus + g.c2h[k]) * cur.uw - mass_x * uo) / msfuy : cur.uw;
+      double u = uw0 + dts * cur.ut;
       double ph_term = (phc1 - phw1) + (phc - phw);
       double p_term = (cur.altw + altc) * (pck - cur.pw);
       double pb_term = (cur.alw + alc) * (pbc - cur.pbw);
@@ -238,8 +264,9 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
     if (do_v) {
       const double phs1 = cur.phs1;
       const unsigned q = vq8 + (unsigned)k * vpl8;
-      double v = cur.vw + dts * cur.vt;
       double mass_y = g.c1h[k] * muv + g.c2h[k];
+      const double vw0 = PREP ? ((g.c1h[k] * muvs + g.c2h[k]) * cur.vw - mass_y * vo) / msfvx : cur.vw;
+      double v = vw0 + dts * cur.vt;
       double ph_term = (phc1 - phs1) + (phc - phs);
       double p_term = (cur.alts + altc) * (pck - cur.ps);
       double pb_term = (cur.als + alc) * (pbc - cur.pbs);
@@ -269,10 +296,10 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
   }
 }
 
-template <int BX, int BY, class TT, bool WET, bool RUNS>
-__global__ void __launch_bounds__(BX * BY) k_uv(DGrid g, DState s, DWork w, double dts, int first, int kc) {
+template <int BX, int BY, class TT, bool WET, bool PREP, bool RUNS>
+__global__ void __launch_bounds__(BX * BY) __attribute__((amdgpu_waves_per_eu(3))) k_uv(DGrid g, DState s, DWork w, double dts, int first, int kc) {
   __shared__ double sh[2][BY][7][BX];
-  b_uv<BX, BY, TT, WET, RUNS>(hw_blk(), &sh[0][0][0][0], g, s, w, dts, first, kc);
+  b_uv<BX, BY, TT, WET, PREP, RUNS>(hw_blk(), &sh[0][0][0][0], g, s, w, dts, first, kc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1877,13 +1904,16 @@ hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DS
   constexpr int BX = kUvBx, BY = kUvBy;
   const int kc = run_levels(uv_tiles(g) * kUvBy, g.nz);
   const dim3 uvgrid(uv_tiles(g), runs_of(g.nz, kc));
+  const bool prep = first && w.uv_preps;
+  void (*uv)(DGrid, DState, DWork, double, int, int);
   if (nl.mixed) {
-    WD_TIMED(prof, KID_UV, st, (WD_RUNS(uvgrid.y, k_uv, BX, BY, float, false)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
+    uv = prep ? WD_RUNS(uvgrid.y, k_uv, BX, BY, float, false, true) : WD_RUNS(uvgrid.y, k_uv, BX, BY, float, false, false);
   } else if (w.cqu) {
-    WD_TIMED(prof, KID_UV, st, (WD_RUNS(uvgrid.y, k_uv, BX, BY, double, true)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
+    uv = prep ? WD_RUNS(uvgrid.y, k_uv, BX, BY, double, true, true) : WD_RUNS(uvgrid.y, k_uv, BX, BY, double, true, false);
   } else {
-    WD_TIMED(prof, KID_UV, st, (WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
+    uv = prep ? WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false, true) : WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false, false);
   }
+  WD_TIMED(prof, KID_UV, st, (uv<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
   // the LDS-tiled kernel has no moisture factor: a moist state runs the column march
   return launch_column_tile(w.cqwr ? kColumnMarch : column_tile, g, nl, s, w, dts, first, st, prof);
 }
@@ -1897,7 +1927,7 @@ hipError_t launch_substep_part(int part, const DGrid& g, const DNamelist& nl, co
   if (part == 0) {
     const int kc = run_levels(uv_tiles(g) * kUvBy, g.nz);
     const dim3 uvgrid(uv_tiles(g), runs_of(g.nz, kc));
-    WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc);
+    WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false, false)<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc);
   } else if (part == 1) {
     k_column_mu<double><<<column_mu_tiles(g), dim3(64, kMuRows), 0, st>>>(g, nl, s, w, dts, first);
   } else if (part == 2) {

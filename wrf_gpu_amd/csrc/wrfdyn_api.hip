@@ -126,6 +126,7 @@ int check_state(wd_handle* h, const wd_state* st, wd::DState* out, int moist_fla
 int enqueue_steps(wd_handle* h, const wd::DState& ds, int n_large_steps, hipStream_t s) {
   const wd::DGrid& g = h->g;
   wd::DWork w = h->w;
+  w.uv_preps = 1;
   // With the column block the stages pass the state on instead of advancing
   // the caller's buffers three times, so the step origin is the caller's state
   // itself and is not copied: stage 1 finishes into `mid`, stage 2 in place,

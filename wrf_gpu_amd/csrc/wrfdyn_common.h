@@ -142,6 +142,8 @@ struct DWork {
   double *cqu, *cqv, *cqwr;
   double* q0[kNumMoist];
   double* qt[kNumMoist];
+  // 1: a stage's first k_uv forms u_work and v_work itself (no k_prep_u/v)
+  int uv_preps;
 };
 
 __host__ __device__ inline size_t im(const DGrid& g, int k, int j, int i) {

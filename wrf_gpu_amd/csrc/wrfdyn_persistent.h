@@ -148,7 +148,7 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
       b_col_setup<TT, false>(tile, lds, M.g, M.nl, M.s, M.w, S.dts);
       break;
     case PK_UV:
-      b_uv<kUvBx, kUvBy, TT, false, false>(tile, lds, M.g, M.s, M.w, S.dts, S.first, 0);
+      b_uv<kUvBx, kUvBy, TT, false, false, false>(tile, lds, M.g, M.s, M.w, S.dts, S.first, 0);
       break;
     case PK_COLUMN_MU:
       b_column_mu<TT>(tile, lds, M.g, M.nl, M.s, M.w, S.dts, S.first);

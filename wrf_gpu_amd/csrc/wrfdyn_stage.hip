@@ -2531,8 +2531,10 @@ hipError_t launch_stage_setup(const DGrid& g, const DNamelist& nl, const DState&
       WD_TIMED(prof, KID_CORIOLIS, st, (launch_coriolis<double>(g, s, w, st)));
   }
   WD_TIMED(prof, KID_PREP_FACES, st, (k_prep_faces<<<blocks_for(F, bs), bs, 0, st>>>(g, w)));
-  WD_TIMED(prof, KID_PREP_U, st, (k_prep_u<<<dim3(blocks_for(CU, bs), kchunks), bs, 0, st>>>(g, s, w)));
-  WD_TIMED(prof, KID_PREP_V, st, (k_prep_v<<<dim3(blocks_for(CV, bs), kchunks), bs, 0, st>>>(g, s, w)));
+  if (!w.uv_preps) {
+    WD_TIMED(prof, KID_PREP_U, st, (k_prep_u<<<dim3(blocks_for(CU, bs), kchunks), bs, 0, st>>>(g, s, w)));
+    WD_TIMED(prof, KID_PREP_V, st, (k_prep_v<<<dim3(blocks_for(CV, bs), kchunks), bs, 0, st>>>(g, s, w)));
+  }
   const unsigned row_tiles = (unsigned)((g.nx + kColOwned - 1) / kColOwned) * (unsigned)g.ny;
   if (bw > 0 && row_tiles <= kFewBlocks / 2) {
     const dim3 block(64, bw);
