@@ -76,3 +76,41 @@ def test_mixed_column_block_matches_the_march():
         dyn.close()
     for k in FIELDS:
         assert np.array_equal(out[0][k], out[1][k]), k
+
+
+@pytest.mark.parametrize("form", ["dry", "moist", "mixed"])
+def test_the_march_choice_runs_the_march(oracle_lib, monkeypatch, form):
+    """WRFDYN_COLUMN_TILE=march selects the column march on a grid that the block holds, in every
+    form and beside a choice of the workgroup order; without it the same grid runs the block."""
+    import torch
+    from wrf_gpu_amd import ic
+    from wrf_gpu_amd.dycore import Dycore, state_to_device, state_to_host
+
+    case = _case(63, 5, 50)
+    if form == "moist":
+        case = ic.with_moisture(case, moist_adv_opt=2)
+    fields = FIELDS + (SPECIES if form == "moist" else ())
+    names = ["k_column_block", "k_column_mu", "k_column_w"]
+    out = {}
+    for choice in ("march", ""):
+        print(f"[block] 63x5x50 {form} WRFDYN_COLUMN_TILE={choice!r}", flush=True)
+        monkeypatch.setenv("WRFDYN_COLUMN_TILE", choice)
+        dyn = Dycore(case.metrics, case.namelist, precision="mixed" if form == "mixed" else "fp64")
+        if choice == "march":
+            dyn.set_tuned_config(-1, 0)
+        st = state_to_device(case.state, "cuda")
+        dyn.profile(names)
+        dyn.step(st, 1)
+        torch.cuda.synchronize()
+        counts = {k: n for k, (_, n) in dyn.profile_read().items()}
+        dyn.close()
+        out[choice] = state_to_host(st)
+        substeps = 1 + 2 + 4
+        want = {"k_column_mu": substeps, "k_column_w": substeps} if choice else {"k_column_block": substeps}
+        assert counts == want, counts
+    for k in fields:
+        assert np.array_equal(out["march"][k], out[""][k]), k
+    if form != "mixed":
+        ref = oracle_lib.run(case.metrics, case.namelist, case.state, 1)
+        for k in fields:
+            assert np.array_equal(out["march"][k], ref[k]), k

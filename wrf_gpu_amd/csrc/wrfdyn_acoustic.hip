@@ -1858,11 +1858,12 @@ const int kNumColumnTiles = sizeof(kColumnTiles) / sizeof(kColumnTiles[0]);
 
 namespace {
 
-hipError_t launch_column_tile(int tile, const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
-                              double dts, int first, hipStream_t st, Prof* prof) {
-  if (tile == kColumnMarch && column_block_waves(g.nz) > 0) {
+hipError_t launch_column(int column, const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
+                         double dts, int first, hipStream_t st, Prof* prof) {
+  if (column == kColumnBlock) {
     const unsigned grid = column_block_tiles(g);
     const int kt = column_block_waves(g.nz);
+    if (kt == 0) return hipErrorInvalidValue;
     const size_t lds = column_block_lds(g.nz, kt) * sizeof(double);
     const dim3 block(64, kt);
     if (nl.mixed)
@@ -1873,7 +1874,7 @@ hipError_t launch_column_tile(int tile, const DGrid& g, const DNamelist& nl, con
       WD_TIMED(prof, KID_COLUMN_BLOCK, st, (k_column_block<kBlockLevels, double, false><<<grid, block, lds, st>>>(g, nl, s, w, dts, first)));
     return hipGetLastError();
   }
-  if (tile == kColumnMarch) {
+  if (column == kColumnMarch) {
     const unsigned bs = 256;
     const size_t C = (size_t)g.ny * g.nx;
     const unsigned mu_tiles = column_mu_tiles(g);
@@ -1889,7 +1890,7 @@ hipError_t launch_column_tile(int tile, const DGrid& g, const DNamelist& nl, con
   }
   // the LDS-tiled kernel reads FP64 tendencies only
   if (nl.mixed) return hipErrorInvalidValue;
-  switch (tile) {
+  switch (column) {
     case 1: return launch_column_levels<8, 16>(g, nl, s, w, dts, first, st, prof);
     case 2: return launch_column_levels<32, 8>(g, nl, s, w, dts, first, st, prof);
     case 3: return launch_column_levels<16, 8>(g, nl, s, w, dts, first, st, prof);
@@ -1900,7 +1901,7 @@ hipError_t launch_column_tile(int tile, const DGrid& g, const DNamelist& nl, con
 }  // namespace
 
 hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
-                                   double dts, int first, int column_tile, hipStream_t st, Prof* prof) {
+                                   double dts, int first, int column, hipStream_t st, Prof* prof) {
   constexpr int BX = kUvBx, BY = kUvBy;
   const int kc = run_levels(uv_tiles(g) * kUvBy, g.nz);
   const dim3 uvgrid(uv_tiles(g), runs_of(g.nz, kc));
@@ -1914,8 +1915,8 @@ hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DS
     uv = prep ? WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false, true) : WD_RUNS(uvgrid.y, k_uv, BX, BY, double, false, false);
   }
   WD_TIMED(prof, KID_UV, st, (uv<<<uvgrid, dim3(BX, BY), 0, st>>>(g, s, w, dts, first, kc)));
-  // the LDS-tiled kernel has no moisture factor: a moist state runs the column march
-  return launch_column_tile(w.cqwr ? kColumnMarch : column_tile, g, nl, s, w, dts, first, st, prof);
+  // the LDS-tiled kernel has no moisture factor: a moist state never runs it
+  return launch_column(w.cqwr && column >= 0 ? kColumnMarch : column, g, nl, s, w, dts, first, st, prof);
 }
 
 hipError_t launch_substep_part(int part, const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,

@@ -35,7 +35,10 @@ struct wd_handle {
   void* diff_buf = nullptr;  // arrays of the optional terms (explicit diffusion, the theta limiter)
   size_t metric_bytes = 0;
   int device = 0;
-  int column_tile = 0;
+  // the LDS tile shape of the acoustic column, or -1: the column block where
+  // it holds the grid's levels, else the column march
+  int column_tile = -1;
+  bool march = false;  // WRFDYN_COLUMN_TILE=march: -1 is the column march at any depth
   std::string err;
   wd::Prof prof;
   // wd_capture_graph: one captured large step and the stream it is captured on
@@ -64,7 +67,7 @@ struct wd_batch {
   // share one device allocation
   bool persistent = false;
   unsigned grid = 0;
-  std::vector<int> column_kernel;  // per member: kColumnMarch or the tile it runs
+  std::vector<int> tiles;  // per member: the LDS tile it runs, or -1
   void* pbuf = nullptr;
   wd::PBarrier* bar = nullptr;
 };
@@ -119,6 +122,12 @@ int check_state(wd_handle* h, const wd_state* st, wd::DState* out, int moist_fla
   return WD_OK;
 }
 
+// The acoustic column kernel the handle's steps run.
+int column_kernel(const wd_handle& h) {
+  if (h.column_tile >= 0) return h.column_tile;
+  return !h.march && wd::column_block_waves(h.g.nz) > 0 ? wd::kColumnBlock : wd::kColumnMarch;
+}
+
 // Enqueue n large steps of _rk_scan_step (operational_mode.py:3319-3534) on
 // stream s: no host synchronisation, allocation or memset, so the sequence
 // can also be captured into a graph (profiling records events, so it is
@@ -133,7 +142,8 @@ int enqueue_steps(wd_handle* h, const wd::DState& ds, int n_large_steps, hipStre
   // stage 3 back into the caller's buffers.  mid is the origin copies' arrays
   // and four that only the other column kernels use (a, alpha, the phi rhs and
   // the forward-swept w; k_col_setup leaves a null a and alpha out).
-  const bool block = h->column_tile == wd::kColumnMarch && wd::column_block_waves(g.nz) > 0;
+  const int column = column_kernel(*h);
+  const bool block = column == wd::kColumnBlock;
   wd::DState mid = ds;
   if (block) {
     mid.u = w.u0;
@@ -200,7 +210,7 @@ int enqueue_steps(wd_handle* h, const wd::DState& ds, int n_large_steps, hipStre
       e = wd::launch_stage_setup(g, h->nl, in, w, sd.rk_step, sd.dts, s, prof);
       if (e != hipSuccess) return hip_fail(h, e, "stage setup launch");
       for (int it = 0; it < sd.nsub; ++it) {
-        e = wd::launch_acoustic_substep(g, h->nl, in, w, sd.dts, it == 0, h->column_tile, s, prof);
+        e = wd::launch_acoustic_substep(g, h->nl, in, w, sd.dts, it == 0, column, s, prof);
         if (e != hipSuccess) return hip_fail(h, e, "acoustic substep launch");
       }
       e = wd::launch_stage_finish(g, in, out, w, s, prof);
@@ -669,13 +679,13 @@ int wd_create(const wd_grid* grid, const wd_namelist* nl, wd_handle** out) {
     }
     h->work_bytes += d_total;
   }
-  // Acoustic column kernel: the column-march pair (default) or, with
-  // WRFDYN_COLUMN_TILE="TXxKT", the LDS-tiled kernel in one of its compiled
-  // tile shapes (when that shape holds nz + 1 levels).
-  h->column_tile = wd::kColumnMarch;
+  // Acoustic column kernel: the column block up to 63 levels and the
+  // column-march pair above them (default); with WRFDYN_COLUMN_TILE="march"
+  // the pair at any depth, with "TXxKT" the LDS-tiled kernel in one of its
+  // compiled tile shapes (when that shape holds nz + 1 levels).
   if (const char* env = std::getenv("WRFDYN_COLUMN_TILE")) {
     int tx = 0, kt = 0;
-    if (std::strcmp(env, "march") == 0) h->column_tile = wd::kColumnMarch;
+    if (std::strcmp(env, "march") == 0) h->march = true;
     else if (std::sscanf(env, "%dx%d", &tx, &kt) == 2) {
       for (int t = 0; t < wd::kNumColumnTiles; ++t)
         if (wd::kColumnTiles[t].tx == tx && wd::kColumnTiles[t].kt == kt &&
@@ -684,7 +694,7 @@ int wd_create(const wd_grid* grid, const wd_namelist* nl, wd_handle** out) {
     }
   }
   // the LDS-tiled kernel has no moisture factor
-  if (h->nl.moist) h->column_tile = wd::kColumnMarch;
+  if (h->nl.moist) h->column_tile = -1;
   *out = h;
   return WD_OK;
 }
@@ -768,11 +778,11 @@ int wd_autotune(wd_handle* h, const wd_state* st, int trial_steps, void* stream)
   }
   hipEvent_t ev[2] = {nullptr, nullptr};
   const int keep_tile = h->column_tile, keep_remap = h->g.xcd_remap;
-  // candidates: the column-march pair and every LDS tile shape that holds nz + 1 levels, each in
-  // both workgroup orders
+  // candidates: the column block (or march) and every LDS tile shape that holds nz + 1 levels, each
+  // in both workgroup orders
   std::vector<std::pair<int, int>> cand;
   for (int remap = 1; remap >= 0; --remap) {
-    cand.emplace_back(wd::kColumnMarch, remap);
+    cand.emplace_back(-1, remap);
     for (int t = 0; t < wd::kNumColumnTiles && !h->nl.mixed && !h->nl.moist; ++t)
       if (h->g.nz + 1 <= wd::kColumnTiles[t].kt * wd::kMaxLevelsPerThread) cand.emplace_back(t, remap);
   }
@@ -831,13 +841,13 @@ int wd_autotune(wd_handle* h, const wd_state* st, int trial_steps, void* stream)
 int wd_set_tuned_config(wd_handle* h, int column_tile, int xcd_remap) {
   if (!h) return fail(nullptr, WD_EINVAL, "handle is NULL");
   if (xcd_remap != 0 && xcd_remap != 1) return fail(h, WD_EINVAL, "xcd_remap must be 0 or 1");
-  if (column_tile != wd::kColumnMarch) {
+  if (column_tile != -1) {
     if (column_tile < 0 || column_tile >= wd::kNumColumnTiles)
       return fail(h, WD_EINVAL, "column_tile must be -1 or a compiled tile shape index");
     if (h->g.nz + 1 > wd::kColumnTiles[column_tile].kt * wd::kMaxLevelsPerThread)
       return fail(h, WD_EINVAL, "the tile shape does not hold the grid's levels");
     if (h->nl.mixed || h->nl.moist)
-      return fail(h, WD_EINVAL, "the mixed form and moist states run the column march (column_tile -1)");
+      return fail(h, WD_EINVAL, "the mixed form and moist states run the column block or the column march (column_tile -1)");
   }
   h->column_tile = column_tile;
   h->g.xcd_remap = xcd_remap;
@@ -853,8 +863,8 @@ int wd_set_precision(wd_handle* h, int mode) {
   if (mode != WD_PREC_FP64 && mode != WD_PREC_MIXED) return fail(h, WD_EINVAL, "precision must be WD_PREC_FP64 or WD_PREC_MIXED");
   if (mode == WD_PREC_MIXED && h->nl.moist) return fail(h, WD_EINVAL, "the mixed form runs dry states only");
   h->nl.mixed = mode == WD_PREC_MIXED;
-  // the mixed form runs the column-march kernels (the LDS-tiled kernel reads FP64 tendencies)
-  if (h->nl.mixed) h->column_tile = wd::kColumnMarch;
+  // the LDS-tiled kernel reads FP64 tendencies
+  if (h->nl.mixed) h->column_tile = -1;
   if (h->graph) {  // a captured graph holds the previous form's kernels
     hipGraphExecDestroy(h->graph);
     h->graph = nullptr;
@@ -944,21 +954,21 @@ int wd_batch_create_persistent(wd_handle* const* members, const wd_state* states
   for (int m = 0; m < n_members; ++m)
     if (members[m]->device != dev) return fail(nullptr, WD_EINVAL, "members must live on the current device");
   std::vector<wd::PMember> pm(n_members);
-  std::vector<int> tiles(n_members);
+  std::vector<int> columns(n_members);
   for (int m = 0; m < n_members; ++m) {
     wd::DState ds;
     int rc = check_state(nullptr, &states[m], &ds, members[m]->nl.moist);
     if (rc != WD_OK) return rc;
     pm[m] = wd::PMember{members[m]->g, members[m]->nl, ds, members[m]->w};
-    tiles[m] = members[m]->column_tile;
+    columns[m] = column_kernel(*members[m]);
   }
-  std::vector<int> column_kernel(n_members);
+  std::vector<int> tiles(n_members);
   for (int m = 0; m < n_members; ++m)
-    column_kernel[m] = wd::persistent_column_levels(pm[m].g, pm[m].nl, tiles[m]) > 0 ? tiles[m] : wd::kColumnMarch;
+    tiles[m] = wd::persistent_column_levels(pm[m].g, pm[m].nl, columns[m]) > 0 ? columns[m] : -1;
   std::vector<wd::PSeg> segs;
   std::vector<wd::PPhase> phases;
   std::string why;
-  if (!wd::persistent_program(pm, tiles, &segs, &phases, &why)) return fail(nullptr, WD_EINVAL, why);
+  if (!wd::persistent_program(pm, columns, &segs, &phases, &why)) return fail(nullptr, WD_EINVAL, why);
   const bool mixed = pm[0].nl.mixed != 0;
   const wd::PForm form = wd::persistent_form(segs);
   // as many workgroups as the GPU holds at once (the grid barrier needs every
@@ -980,7 +990,7 @@ int wd_batch_create_persistent(wd_handle* const* members, const wd_state* states
   b->device = dev;
   b->persistent = true;
   b->grid = grid;
-  b->column_kernel = column_kernel;
+  b->tiles = tiles;
   b->members.assign(members, members + n_members);
   b->states.resize(n_members);
   for (int m = 0; m < n_members; ++m) b->states[m] = pm[m].s;
@@ -1077,7 +1087,7 @@ int wd_batch_workgroups(const wd_batch* b) { return b ? (int)b->grid : WD_EINVAL
 
 int wd_batch_column_kernel(const wd_batch* b, int member, int* column_tile) {
   if (!b || !column_tile || member < 0 || member >= (int)b->members.size()) return WD_EINVAL;
-  *column_tile = b->persistent ? b->column_kernel[member] : b->members[member]->column_tile;
+  *column_tile = b->persistent ? b->tiles[member] : b->members[member]->column_tile;
   return WD_OK;
 }
 
@@ -1236,7 +1246,6 @@ int wd_step_noalloc(const wd_grid* grid, const wd_namelist* nl, const wd_state* 
   if (rc != WD_OK) return rc;
   wd_handle h;  // on the stack: its device buffers all come from `scratch`
   init_params(grid, nl, rot, h.g, h.nl);
-  h.column_tile = wd::kColumnMarch;
   // the layout in `scratch`: the metrics, then the workspace (base, then the
   // optional terms' arrays), each 256-byte aligned
   const size_t n1 = grid->nz, n1f = (size_t)grid->nz + 1;

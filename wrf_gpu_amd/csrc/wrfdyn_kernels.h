@@ -110,16 +110,18 @@ struct ColumnTile {
   int tx, kt;
 };
 constexpr int kMaxLevelsPerThread = 8;
-// column_tile value that selects the column-march kernel instead of a tile shape
-constexpr int kColumnMarch = -1;
+// The acoustic column kernel of a step: a tile shape's index, or one of these
+constexpr int kColumnMarch = -1;  // the march pair k_column_mu + k_column_w
+constexpr int kColumnBlock = -2;  // k_column_block (column_block_waves(nz) > 0)
 extern const ColumnTile kColumnTiles[];
 extern const int kNumColumnTiles;
 
-// One acoustic substep: advance_uv, then the fused column kernel with tile
-// shape kColumnTiles[column_tile].  `first` marks a stage's first substep,
-// which starts from t_2ave = 0 and pm1 = the step-0 pressure.
+// One acoustic substep: advance_uv, then the column kernel `column`
+// (kColumnBlock, kColumnMarch or a kColumnTiles index).  `first` marks a
+// stage's first substep, which starts from t_2ave = 0 and pm1 = the step-0
+// pressure.
 hipError_t launch_acoustic_substep(const DGrid& g, const DNamelist& nl, const DState& s, const DWork& w,
-                                   double dts, int first, int column_tile, hipStream_t st, Prof* prof);
+                                   double dts, int first, int column, hipStream_t st, Prof* prof);
 
 // The moisture's large-step update after the acoustic loop of a stage with
 // transport on (moist_adv_opt != 0): q = (m_origin q0 + dt_rk qt) / m_new.
@@ -171,16 +173,18 @@ struct PBarrier {
   unsigned count, gen, abort, spin_limit;
 };
 // The program of one large step of the members (all of one precision form
-// and one substep count; no optional term but rotation).  column_tiles holds
-// each member's acoustic column kernel (kColumnMarch or a kColumnTiles index):
-// the 16 x 16 tile runs as such for up to 63 levels in the FP64 form, any
-// other choice as the column march, which gives the same bits.  Returns false
-// with a message for a member it cannot run.
-bool persistent_program(const std::vector<PMember>& members, const std::vector<int>& column_tiles,
+// and one substep count; no optional term but rotation).  columns holds each
+// member's acoustic column kernel (kColumnBlock, kColumnMarch or a
+// kColumnTiles index): the 16 x 16 tile runs as such for up to 63 levels in
+// the FP64 form; any other choice but kColumnMarch runs as the column block
+// in a small ensemble without tiles (persistent_program tells the limits);
+// the rest as the column march.  All give the same bits.  Returns false with
+// a message for a member it cannot run.
+bool persistent_program(const std::vector<PMember>& members, const std::vector<int>& columns,
                         std::vector<PSeg>* segs, std::vector<PPhase>* phases, std::string* why);
 // Levels per thread with which the persistent step runs a member's column
-// tile, 0 where it runs the column march.
-int persistent_column_levels(const DGrid& g, const DNamelist& nl, int column_tile);
+// tile, 0 where it runs the column block or march.
+int persistent_column_levels(const DGrid& g, const DNamelist& nl, int column);
 // The persistent kernel a program runs: with the column march, with the column
 // tile beside it (FP64), or with the column block (a small ensemble).
 enum class PForm { march, tile, block };

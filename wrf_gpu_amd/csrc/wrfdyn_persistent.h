@@ -307,31 +307,33 @@ __global__ void __launch_bounds__(256) k_step_persistent_block(const PMember* __
 
 }  // namespace
 
-int persistent_column_levels(const DGrid& g, const DNamelist& nl, int column_tile) {
-  if (column_tile != kPersistTile || nl.mixed) return 0;
+int persistent_column_levels(const DGrid& g, const DNamelist& nl, int column) {
+  if (column != kPersistTile || nl.mixed) return 0;
   const int r = (g.nz + 1 + kPersistTileKt - 1) / kPersistTileKt;
   return r <= kPersistTileLevels ? r : 0;
 }
 
-bool persistent_program(const std::vector<PMember>& members, const std::vector<int>& column_tiles,
+bool persistent_program(const std::vector<PMember>& members, const std::vector<int>& columns,
                         std::vector<PSeg>* segs, std::vector<PPhase>* phases, std::string* why) {
   segs->clear();
   phases->clear();
-  if (members.empty() || column_tiles.size() != members.size()) {
+  if (members.empty() || columns.size() != members.size()) {
     *why = members.empty() ? "no members" : "one column kernel choice per member";
     return false;
   }
   const int nm = (int)members.size();
-  // levels per thread of the member's LDS column tile, 0 for the column march
+  // levels per thread of the member's LDS column tile, 0 without
   std::vector<int> tile_levels(nm);
-  for (int m = 0; m < nm; ++m) tile_levels[m] = persistent_column_levels(members[m].g, members[m].nl, column_tiles[m]);
+  for (int m = 0; m < nm; ++m) tile_levels[m] = persistent_column_levels(members[m].g, members[m].nl, columns[m]);
   const bool any_tile = std::count(tile_levels.begin(), tile_levels.end(), 0) < nm;
   // the column block instead of the march, where the launch is short of waves
+  // (and the member was not held to the march)
   std::vector<char> use_block(nm, 0);
   unsigned long long block_tiles = 0;
   for (const PMember& m : members) block_tiles += column_block_tiles(m.g);
   for (int m = 0; m < nm; ++m)
-    use_block[m] = !any_tile && block_tiles <= kPersistBlockTiles && members[m].g.nz <= kPersistBlockNz;
+    use_block[m] = !any_tile && columns[m] != kColumnMarch && block_tiles <= kPersistBlockTiles &&
+                   members[m].g.nz <= kPersistBlockNz;
   bool any_march = false;
   for (int m = 0; m < nm; ++m) any_march = any_march || (tile_levels[m] == 0 && !use_block[m]);
   const DNamelist& n0 = members[0].nl;
