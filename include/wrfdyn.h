@@ -160,12 +160,21 @@ int wd_graph_step(wd_handle *h, int n_large_steps, void *stream);
  * in the large-step pressure gradient, calc_p_rho, advance_w's pressure and
  * buoyancy terms and rw_tend, the tridiagonal solve and the mu/theta
  * accumulation.  Results then differ from the FP64 form by rounding-level
- * amounts; they are not bit-identical.  The mixed form runs the column-march
- * kernels.  Changing the form drops a captured graph. */
+ * amounts; they are not bit-identical.  The mixed form runs the column block
+ * or march, never an LDS tile.  Changing the form drops a captured graph. */
 #define WD_PREC_FP64 0
 #define WD_PREC_MIXED 1
 int wd_set_precision(wd_handle *h, int mode);
 int wd_get_precision(const wd_handle *h);
+
+/* The acoustic column kernels.  All give identical results.  A handle runs,
+ * unless it is tuned to an LDS tile shape, the column block (one launch a
+ * substep, a workgroup holding its columns' levels in registers) up to 63
+ * levels and the column march (two launches) above them.  The environment
+ * variable WRFDYN_COLUMN_TILE, read by wd_create, picks another kernel:
+ * "march" the column march at any depth, "TXxKT" a tile shape. */
+#define WD_COLUMN_MARCH (-1)
+#define WD_COLUMN_BLOCK (-2)
 
 /* Tile-shape autotuner (no counterpart in the reference, which leaves launch
  * shapes to XLA).  Times every compiled form of the acoustic column kernel
@@ -173,15 +182,15 @@ int wd_get_precision(const wd_handle *h);
  * order, over `trial_steps` large steps each on a scratch copy of `state`
  * (allocated and freed here; the caller's state is not changed), and keeps
  * the fastest for later steps.  Synchronises `stream`.  All forms give
- * identical results.  wd_tuned_config reports the choice: column_tile -1 is
- * the column-march kernel pair, t >= 0 the t-th LDS tile shape.  In the mixed
- * form only the workgroup order is tuned. */
+ * identical results.  wd_tuned_config reports the choice: column_tile -1 is no
+ * tile (the column block or march, as above), t >= 0 the t-th LDS tile shape.
+ * In the mixed form and with moisture only the workgroup order is tuned. */
 int wd_autotune(wd_handle *h, const wd_state *state, int trial_steps, void *stream);
 int wd_tuned_config(const wd_handle *h, int *column_tile, int *xcd_remap);
 /* Applies a tuning (a saved wd_tuned_config, or a choice of the caller's):
  * WD_EINVAL for a tile shape that does not hold the grid's levels, or any
- * tile in the mixed form or with moisture, which run the column march.  A
- * captured graph is dropped.  No reference counterpart. */
+ * tile in the mixed form or with moisture, which run the column block or
+ * march.  A captured graph is dropped.  No reference counterpart. */
 int wd_set_tuned_config(wd_handle *h, int column_tile, int xcd_remap);
 
 /* Ensembles of independent members with differing grids (no counterpart in
@@ -214,10 +223,12 @@ int wd_batch_branches(const wd_batch *b);
  * the precision form and the substep count and use none of the explicit
  * diffusions, the limiter or the moisture (WD_EINVAL).  Each member keeps
  * its tuned workgroup order and, in the FP64 form up to 63 levels, a tuned
- * 16 x 16 LDS column tile; any other column form runs as the column march,
- * which gives the same bits (wd_batch_column_kernel tells which runs).  The grid barrier needs every workgroup resident,
- * so nothing else may run on the GPU during a persistent step: a barrier
- * wait that runs out of polls (wd_batch_set_spin_limit) abandons the step
+ * 16 x 16 LDS column tile; any other column form runs as the column block,
+ * for members of up to 51 levels in a small ensemble (at most 512 column
+ * blocks of 62 columns of a row) without such tiles, and as the column march
+ * elsewhere, with the same bits (wd_batch_column_form tells which runs).  The
+ * grid barrier needs every workgroup resident, so nothing else may run on
+ * the GPU during a persistent step: a barrier wait that runs out of polls (wd_batch_set_spin_limit) abandons the step
  * and every later one until wd_batch_status reports it.  wd_batch_branches
  * is 1 and wd_batch_workgroups gives the launch's workgroup count. */
 int wd_batch_create_persistent(wd_handle *const *members, const wd_state *states, int n_members,
@@ -230,12 +241,15 @@ int wd_batch_status(wd_batch *b, void *stream);
  * (default 4,194,304).  Synchronises the device. */
 int wd_batch_set_spin_limit(wd_batch *b, unsigned polls);
 int wd_batch_workgroups(const wd_batch *b);
-/* The acoustic column kernel that `member` runs in the batch's step: -1 for
- * the column march, else the index of its LDS tile shape (as
- * wd_tuned_config).  For a graph batch this is the member's own choice; a
- * persistent batch reports what its step runs.  No reference counterpart: a
- * query of this build's batched forms. */
+/* The LDS tile shape that `member` runs in the batch's step (an index as in
+ * wd_tuned_config), or -1 where it runs none.  For a graph batch this is the
+ * member's own choice; a persistent batch reports what its step runs.  No
+ * reference counterpart: a query of this build's batched forms. */
 int wd_batch_column_kernel(const wd_batch *b, int member, int *column_tile);
+/* The acoustic column kernel that the batch's captured step runs for
+ * `member`: WD_COLUMN_BLOCK, WD_COLUMN_MARCH or the index of its LDS tile
+ * shape. */
+int wd_batch_column_form(const wd_batch *b, int member, int *form);
 
 const char *wd_batch_last_error(const wd_batch *b);
 void wd_batch_destroy(wd_batch *b);

@@ -70,17 +70,19 @@ def _dycore(case, precision, column=None):
             os.environ["WRFDYN_COLUMN_TILE"] = keep
 
 
-def _run_pair(cases, steps, precision="fp64", columns=None, expect_kernels=None, remaps=None):
+def _run_pair(cases, steps, precision="fp64", columns=None, expect_kernels=None, remaps=None, expect_forms=None,
+              alone_columns=None):
     """Each case stepped alone and in one persistent ensemble; returns both host states per case.
-    ``columns`` gives each member's column kernel choice, ``expect_kernels`` the column kernel
-    the persistent step must then run for each (-1 the column march, 0 the 16x16 tile), and
+    ``columns`` gives each member's column kernel choice (``alone_columns`` that of the case stepped
+    alone, where it differs), ``expect_kernels`` the tile the persistent step must then run for each
+    (-1 none, 0 the 16x16 tile), ``expect_forms`` the column kernel ("block", "march" or "tile"), and
     ``remaps`` each member's workgroup order (1 XCD-contiguous, 0 hardware order)."""
 
     import torch
     from wrf_gpu_amd.dycore import Ensemble, state_to_device, state_to_host
 
     columns = columns or [None] * len(cases)
-    alone = [(_dycore(c, precision, col), state_to_device(c.state)) for c, col in zip(cases, columns)]
+    alone = [(_dycore(c, precision, col), state_to_device(c.state)) for c, col in zip(cases, alone_columns or columns)]
     batched = [(_dycore(c, precision, col), state_to_device(c.state)) for c, col in zip(cases, columns)]
     for m, remap in enumerate(remaps or []):
         for d, _ in (alone[m], batched[m]):
@@ -90,8 +92,11 @@ def _run_pair(cases, steps, precision="fp64", columns=None, expect_kernels=None,
     kernels = [ens.column_kernel(m) for m in range(len(cases))]
     if expect_kernels is not None:
         assert kernels == list(expect_kernels), kernels
+    forms = [ens.column_form(m) for m in range(len(cases))]
+    if expect_forms is not None:
+        assert forms == list(expect_forms), forms
     print(f"[persistent] {len(cases)} members, {precision}, {ens.workgroups} workgroups, steps {steps}, "
-          f"column kernels {kernels}", flush=True)
+          f"column kernels {forms}", flush=True)
     out = []
     done = 0
     for n in steps:
@@ -241,6 +246,51 @@ def test_persistent_mixed_form_keeps_the_column_march():
 
     cases = [ic.stratified_terrain_3d(nx=20, ny=18, nz=40, dx=3000.0, u_sigma=1.0, sigma=0.5)]
     _run_pair(cases, (2,), precision="mixed", columns=["16x16"], expect_kernels=[-1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("grids,forms", [
+    (((21, 7, 51),), ["block"]),
+    (((21, 7, 52),), ["march"]),
+    (((21, 7, 51), (63, 6, 52)), ["block", "march"]),
+    (((62, 512, 4),), ["block"]),
+    (((62, 256, 4), (63, 128, 5)), ["block", "block"]),
+    (((62, 513, 4),), ["march"]),
+    (((62, 256, 4), (63, 129, 5)), ["march", "march"]),
+])
+def test_persistent_on_both_sides_of_the_column_block_limits(oracle_lib, grids, forms, precision):
+    """51 levels, the most that the block's four waves of 13 hold, and 52; a member of each in one
+    launch; 512 column blocks in all, the most for which the step runs them, and just above, in one
+    member and in two.  The members alone run the other column kernel, FP64 also against the oracle."""
+
+    from wrf_gpu_amd import ic
+
+    cases = [ic.stratified_terrain_3d(nx=nx, ny=ny, nz=nz, dx=3000.0, ns=4, u_sigma=1.0, sigma=0.5)
+             for nx, ny, nz in grids]
+    out = _run_pair(cases, (2,), precision=precision, expect_forms=forms,
+                    alone_columns=["march" if f == "block" else None for f in forms])
+    if precision == "fp64":
+        for c, (_, got) in zip(cases, out):
+            ref = oracle_lib.run(c.metrics, c.namelist, c.state, 2)
+            _assert_bitwise(got, ref, c.name)
+
+
+@pytest.mark.parametrize("nz,form", [(63, "block"), (64, "march")])
+def test_graph_ensemble_reports_the_column_kernel(nz, form):
+    """The graph of launches runs the block up to 63 levels, the march above them or where it was
+    chosen, and a tuned tile; ``column_form`` tells."""
+
+    from wrf_gpu_amd import ic
+    from wrf_gpu_amd.dycore import Ensemble, state_to_device
+
+    case = ic.stratified_terrain_3d(nx=12, ny=5, nz=nz, dx=3000.0, u_sigma=1.0, sigma=0.5)
+    members = [(_dycore(case, "fp64", col), state_to_device(case.state)) for col in (None, "march", "16x16")]
+    ens = Ensemble(members)
+    assert [ens.column_form(m) for m in range(3)] == [form, "march", "tile"]
+    assert [ens.column_kernel(m) for m in range(3)] == [-1, -1, 0]
+    ens.close()
+    for d, _ in members:
+        d.close()
 
 
 def test_persistent_at_the_ensemble_member_sizes():

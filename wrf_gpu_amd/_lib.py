@@ -22,6 +22,9 @@ WD_EDEVICE = -3
 WD_PREC_FP64 = 0
 WD_PREC_MIXED = 1
 
+WD_COLUMN_MARCH = -1
+WD_COLUMN_BLOCK = -2
+
 EXPORTED_SYMBOLS = ("wd_create", "wd_step", "wd_workspace_bytes", "wd_last_error", "wd_destroy",
                     "wd_profile_enable", "wd_profile_read", "wd_kernel_count", "wd_kernel_name",
                     "wd_capture_graph", "wd_graph_step", "wd_autotune", "wd_tuned_config", "wd_set_tuned_config",
@@ -29,7 +32,7 @@ EXPORTED_SYMBOLS = ("wd_create", "wd_step", "wd_workspace_bytes", "wd_last_error
                     "wd_batch_create", "wd_step_batched", "wd_batch_branch", "wd_batch_branches",
                     "wd_batch_last_error", "wd_batch_destroy", "wd_step_adjoint", "wd_adjoint_tape_bytes",
                     "wd_step_noalloc", "wd_batch_create_persistent", "wd_batch_status", "wd_batch_set_spin_limit",
-                    "wd_batch_workgroups", "wd_batch_column_kernel")
+                    "wd_batch_workgroups", "wd_batch_column_kernel", "wd_batch_column_form")
 
 
 class WdGrid(ctypes.Structure):
@@ -154,6 +157,8 @@ def load() -> ctypes.CDLL:
         lib.wd_batch_set_spin_limit.argtypes = [ctypes.c_void_p, ctypes.c_uint]
         lib.wd_batch_workgroups.restype = ctypes.c_int
         lib.wd_batch_workgroups.argtypes = [ctypes.c_void_p]
+        lib.wd_batch_column_form.restype = ctypes.c_int
+        lib.wd_batch_column_form.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
         lib.wd_batch_column_kernel.restype = ctypes.c_int
         lib.wd_batch_column_kernel.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
         _lib = lib

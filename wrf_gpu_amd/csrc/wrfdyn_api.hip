@@ -58,6 +58,7 @@ struct wd_batch {
   std::vector<hipStream_t> streams;
   std::vector<hipEvent_t> events;
   std::vector<int> branch_of;  // member -> branch
+  std::vector<int> columns;    // member -> the acoustic column kernel its captured step runs
   int branches = 1;            // branches in use (<= streams.size())
   hipGraphExec_t graph = nullptr;
   int device = 0;
@@ -67,7 +68,6 @@ struct wd_batch {
   // share one device allocation
   bool persistent = false;
   unsigned grid = 0;
-  std::vector<int> tiles;  // per member: the LDS tile it runs, or -1
   void* pbuf = nullptr;
   wd::PBarrier* bar = nullptr;
 };
@@ -903,6 +903,7 @@ int wd_batch_create(wd_handle* const* members, const wd_state* states, int n_mem
   if (!b) return fail(nullptr, WD_ENOMEM, "host allocation failed");
   b->device = dev;
   b->members.assign(members, members + n_members);
+  for (wd_handle* h : b->members) b->columns.push_back(column_kernel(*h));
   b->states.resize(n_members);
   for (int m = 0; m < n_members; ++m) {
     int rc = check_state(nullptr, &states[m], &b->states[m], members[m]->nl.moist);
@@ -962,9 +963,6 @@ int wd_batch_create_persistent(wd_handle* const* members, const wd_state* states
     pm[m] = wd::PMember{members[m]->g, members[m]->nl, ds, members[m]->w};
     columns[m] = column_kernel(*members[m]);
   }
-  std::vector<int> tiles(n_members);
-  for (int m = 0; m < n_members; ++m)
-    tiles[m] = wd::persistent_column_levels(pm[m].g, pm[m].nl, columns[m]) > 0 ? columns[m] : -1;
   std::vector<wd::PSeg> segs;
   std::vector<wd::PPhase> phases;
   std::string why;
@@ -990,7 +988,8 @@ int wd_batch_create_persistent(wd_handle* const* members, const wd_state* states
   b->device = dev;
   b->persistent = true;
   b->grid = grid;
-  b->tiles = tiles;
+  for (int m = 0; m < n_members; ++m) columns[m] = wd::persistent_column(segs, m);
+  b->columns = columns;
   b->members.assign(members, members + n_members);
   b->states.resize(n_members);
   for (int m = 0; m < n_members; ++m) b->states[m] = pm[m].s;
@@ -1087,7 +1086,14 @@ int wd_batch_workgroups(const wd_batch* b) { return b ? (int)b->grid : WD_EINVAL
 
 int wd_batch_column_kernel(const wd_batch* b, int member, int* column_tile) {
   if (!b || !column_tile || member < 0 || member >= (int)b->members.size()) return WD_EINVAL;
-  *column_tile = b->persistent ? b->tiles[member] : b->members[member]->column_tile;
+  if (b->persistent) *column_tile = b->columns[member] >= 0 ? b->columns[member] : -1;
+  else *column_tile = b->members[member]->column_tile;
+  return WD_OK;
+}
+
+int wd_batch_column_form(const wd_batch* b, int member, int* form) {
+  if (!b || !form || member < 0 || member >= (int)b->members.size()) return WD_EINVAL;
+  *form = b->columns[member];
   return WD_OK;
 }
 

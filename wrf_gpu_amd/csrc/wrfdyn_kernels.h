@@ -6,6 +6,7 @@
 #include <utility>
 #include <vector>
 
+#include "wrfdyn.h"
 #include "wrfdyn_common.h"
 
 namespace wd {
@@ -111,8 +112,8 @@ struct ColumnTile {
 };
 constexpr int kMaxLevelsPerThread = 8;
 // The acoustic column kernel of a step: a tile shape's index, or one of these
-constexpr int kColumnMarch = -1;  // the march pair k_column_mu + k_column_w
-constexpr int kColumnBlock = -2;  // k_column_block (column_block_waves(nz) > 0)
+constexpr int kColumnMarch = WD_COLUMN_MARCH;  // the march pair k_column_mu + k_column_w
+constexpr int kColumnBlock = WD_COLUMN_BLOCK;  // k_column_block (column_block_waves(nz) > 0)
 extern const ColumnTile kColumnTiles[];
 extern const int kNumColumnTiles;
 
@@ -182,9 +183,9 @@ struct PBarrier {
 // a message for a member it cannot run.
 bool persistent_program(const std::vector<PMember>& members, const std::vector<int>& columns,
                         std::vector<PSeg>* segs, std::vector<PPhase>* phases, std::string* why);
-// Levels per thread with which the persistent step runs a member's column
-// tile, 0 where it runs the column block or march.
-int persistent_column_levels(const DGrid& g, const DNamelist& nl, int column);
+// The column kernel that a program runs for a member: kColumnBlock,
+// kColumnMarch or a kColumnTiles index.
+int persistent_column(const std::vector<PSeg>& segs, int member);
 // The persistent kernel a program runs: with the column march, with the column
 // tile beside it (FP64), or with the column block (a small ensemble).
 enum class PForm { march, tile, block };

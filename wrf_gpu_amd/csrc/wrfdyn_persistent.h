@@ -307,10 +307,25 @@ __global__ void __launch_bounds__(256) k_step_persistent_block(const PMember* __
 
 }  // namespace
 
+namespace {
+
+// Levels per thread with which the persistent step runs a member's column
+// tile, 0 where it runs the column block or march.
 int persistent_column_levels(const DGrid& g, const DNamelist& nl, int column) {
   if (column != kPersistTile || nl.mixed) return 0;
   const int r = (g.nz + 1 + kPersistTileKt - 1) / kPersistTileKt;
   return r <= kPersistTileLevels ? r : 0;
+}
+
+}  // namespace
+
+int persistent_column(const std::vector<PSeg>& segs, int member) {
+  for (const PSeg& S : segs)
+    if (S.member == member) {
+      if (S.kind == PK_COLUMN_TILE) return kPersistTile;
+      if (S.kind == PK_COLUMN_BLOCK) return kColumnBlock;
+    }
+  return kColumnMarch;
 }
 
 bool persistent_program(const std::vector<PMember>& members, const std::vector<int>& columns,

@@ -211,7 +211,9 @@ class Dycore:
     def autotune(self, state: dict, trial_steps: int = 2, stream=None) -> dict:
         """Time the column-kernel forms and workgroup orders on a copy of ``state``; keep the fastest.
 
-        Returns ``{"column_tile": t, "xcd_remap": r}`` (t = -1: column-march kernels).
+        Returns ``{"column_tile": t, "xcd_remap": r}`` (t = -1: no LDS tile, that is the column block up
+        to 63 levels and the column march above them, or the march at any depth for a handle created
+        with ``WRFDYN_COLUMN_TILE=march``).
         """
 
         self.check_state(state)
@@ -281,9 +283,9 @@ class Ensemble:
     ``tuned`` then lists the choices made alone.  Tuned alone, a member does
     not see the other members running beside it, so if some member picked an
     LDS column tile, the batched step is then timed on copies of the states
-    with those picks and with every member on the column march (same bits),
-    and the faster is kept (``batch_trial``).  Each member keeps its tuned
-    workgroup order.
+    with those picks and with every member off its tile (same bits), and the
+    faster is kept (``batch_trial``).  Each member keeps its tuned workgroup
+    order.
 
     ``persistent=True`` captures instead one launch of the persistent step
     per large step (``wd_batch_create_persistent``): every kernel body of
@@ -291,12 +293,14 @@ class Ensemble:
     that meet at a grid barrier between phases.  With ``autotune=True`` a
     member tuned to the 16x16 LDS column tile runs that tile inside the
     launch (FP64, up to 63 levels; ``column_kernel`` tells), unless the
-    persistent step with every member on the column march is faster: both
+    persistent step with every member off its tile is faster: both
     are timed on copies of the states (``persistent_trial``) and the faster
-    kept.  Members must share the
-    precision form and substep count and use no explicit diffusion, limiter
-    or moisture; nothing else may run on the GPU during a step.  ``status``
-    synchronises and raises if a barrier wait ran out since the last check.
+    kept.  Members without a tile run the column block in a small ensemble
+    and the column march in a large one (``column_form`` tells).  Members
+    must share the precision form and substep count and use no explicit
+    diffusion, limiter or moisture; nothing else may run on the GPU during a
+    step.  ``status`` synchronises and raises if a barrier wait ran out since
+    the last check.
     """
 
     def __init__(self, members, branches: int = 4, autotune: bool = False, trial_steps: int = 1,
@@ -338,9 +342,9 @@ class Ensemble:
 
     def _batch_trial(self, trial_steps: int, persistent: bool, branches: int) -> dict:
         """Time the batched step (the persistent step, or the graph on ``branches`` branches) with the
-        members' own tuned column tiles and with every member on the column march (same bits), on
-        copies of the states, and keep the faster: each member was tuned alone, without the other
-        members beside it or the persistent kernel's occupancy."""
+        members' own tuned column tiles and with every member off its tile (``march_ms``: the column
+        block or march, same bits), on copies of the states, and keep the faster: each member was tuned
+        alone, without the other members beside it or the persistent kernel's occupancy."""
 
         import torch
 
@@ -379,11 +383,18 @@ class Ensemble:
         return int(self._lib.wd_batch_workgroups(self._batch))
 
     def column_kernel(self, member: int) -> int:
-        """The acoustic column kernel ``member`` runs in the ensemble's step: -1 the column march, else a tile index."""
+        """The LDS tile shape ``member`` runs in the ensemble's step, or -1 where it runs none."""
 
         out = ctypes.c_int(0)
         self._check(self._lib.wd_batch_column_kernel(self._batch, int(member), ctypes.byref(out)))
         return out.value
+
+    def column_form(self, member: int) -> str:
+        """The acoustic column kernel ``member`` runs in the ensemble's step: "block", "march" or "tile"."""
+
+        out = ctypes.c_int(0)
+        self._check(self._lib.wd_batch_column_form(self._batch, int(member), ctypes.byref(out)))
+        return {_lib.WD_COLUMN_BLOCK: "block", _lib.WD_COLUMN_MARCH: "march"}.get(out.value, "tile")
 
     def status(self, stream=None) -> None:
         """Synchronise ``stream``; raise if a persistent step's barrier wait ran out since the last call."""
