@@ -3,8 +3,11 @@ the CPU oracle at the sizes where its tiling can go wrong: the column counts aro
 workgroups, one row, the fewest levels, level counts that leave the last wave one to four
 levels, the deepest grid it takes (63 levels) and the first that runs the column march instead
 (64).  Every value is computed by the oracle's operations in the oracle's order, so the
-comparison is exact.  The mixed form is compared with the persistent step, which runs the
-column march's kernels in the same precision form."""
+comparison is exact.  The mixed form, which has no oracle, is compared with the column march
+in the same precision form.  The damping of w where the vertical Courant number exceeds 1 is
+run by winds that reach it."""
+
+import dataclasses
 
 import numpy as np
 import pytest
@@ -55,27 +58,37 @@ def test_moist_column_block_matches_oracle(oracle_lib):
         assert np.array_equal(got[k], ref[k]), k
 
 
-def test_mixed_column_block_matches_the_march():
+def test_mixed_column_block_matches_the_march(monkeypatch):
+    """The block of the eager step (four levels a wave) and of the persistent step (13) against the
+    march in both, mixed form; the persistent ones say which they ran, the eager one's launches are
+    counted."""
     import torch
     from wrf_gpu_amd.dycore import Dycore, Ensemble, state_to_device, state_to_host
 
     case = _case(63, 5, 50)
-    out = []
-    for persistent in (False, True):
-        st = state_to_device(case.state, "cuda")
-        dyn = Dycore(case.metrics, case.namelist, precision="mixed")
-        if persistent:
-            ens = Ensemble([(dyn, st)], persistent=True)
-            ens.step(2)
-            ens.status()
-            ens.close()
-        else:
-            dyn.step(st, 2)
-        torch.cuda.synchronize()
-        out.append(state_to_host(st))
-        dyn.close()
-    for k in FIELDS:
-        assert np.array_equal(out[0][k], out[1][k]), k
+    out = {}
+    for choice in ("block", "march"):
+        monkeypatch.setenv("WRFDYN_COLUMN_TILE", "" if choice == "block" else choice)
+        for persistent in (False, True):
+            print(f"[block] 63x5x50 mixed {choice} persistent={persistent}", flush=True)
+            st = state_to_device(case.state, "cuda")
+            dyn = Dycore(case.metrics, case.namelist, precision="mixed")
+            if persistent:
+                ens = Ensemble([(dyn, st)], persistent=True)
+                assert ens.column_form(0) == choice
+                ens.step(2)
+                ens.status()
+                ens.close()
+            else:
+                dyn.profile(["k_column_block", "k_column_w"])
+                dyn.step(st, 2)
+                assert list(dyn.profile_read()) == ["k_column_block" if choice == "block" else "k_column_w"]
+            torch.cuda.synchronize()
+            out[choice, persistent] = state_to_host(st)
+            dyn.close()
+    for key, got in out.items():
+        for k in FIELDS:
+            assert np.array_equal(got[k], out["march", False][k]), (key, k)
 
 
 @pytest.mark.parametrize("form", ["dry", "moist", "mixed"])
@@ -114,3 +127,39 @@ def test_the_march_choice_runs_the_march(oracle_lib, monkeypatch, form):
         ref = oracle_lib.run(case.metrics, case.namelist, case.state, 1)
         for k in fields:
             assert np.array_equal(out["march"][k], ref[k]), k
+
+
+@pytest.mark.parametrize("nz,column,persistent", [(47, "", False), (63, "", False), (47, "", True), (47, "march", False),
+                                                  (64, "", False), (47, "16x16", False)])
+def test_w_damping_above_a_courant_number_of_one_matches_oracle(oracle_lib, monkeypatch, nz, column, persistent):
+    """Winds that diverge from face to face and turn with height drive the vertical Courant number
+    of the acoustic omega above 1 in most columns and leave it below 1 in others."""
+    import torch
+    from wrf_gpu_amd.dycore import Dycore, Ensemble, state_to_device, state_to_host
+
+    base = _case(20, 6, nz)
+    z = (np.arange(nz) + 0.5) / nz
+    state = dict(base.state)
+    state["u"] = state["u"] + 40.0 * np.cos(np.pi * z)[:, None, None] * np.where(np.arange(21) % 2 == 0, 1.0, -1.0)
+    nl = dataclasses.replace(base.namelist, dt_s=12.0, w_damping=1)
+    ref = oracle_lib.run(base.metrics, nl, state, 1)
+    off = oracle_lib.run(base.metrics, dataclasses.replace(nl, w_damping=0), state, 1)
+    acted = ref["w"] != off["w"]
+    assert acted.any() and not acted[1:nz].all()
+    print(f"[block] 20x6x{nz} Courant {column!r} persistent={persistent}", flush=True)
+    monkeypatch.setenv("WRFDYN_COLUMN_TILE", column)
+    dyn = Dycore(base.metrics, nl)
+    st = state_to_device(state, "cuda")
+    if persistent:
+        ens = Ensemble([(dyn, st)], persistent=True)
+        assert ens.column_form(0) == "block"
+        ens.step(1)
+        ens.status()
+        ens.close()
+    else:
+        dyn.step(st, 1)
+    torch.cuda.synchronize()
+    dyn.close()
+    got = state_to_host(st)
+    for k in FIELDS:
+        assert np.array_equal(got[k], ref[k]), k

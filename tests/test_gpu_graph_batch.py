@@ -110,8 +110,8 @@ def test_batched_members_match_individual_steps(oracle_lib, branches):
 
 def test_autotuned_ensemble_matches_members_alone(oracle_lib):
     """Ensemble(autotune=True) tunes every member alone, times the batch with those picks and
-    with every member on the column march, and captures the faster (the LDS-tiled column kernel
-    or the column march, either workgroup order); the states are untouched by the trials, and the
+    with every member off its tile, and captures the faster (the LDS-tiled column kernel
+    or the column block, either workgroup order); the states are untouched by the trials, and the
     result is still bitwise each member stepped alone, a moist member included."""
 
     import torch
@@ -128,7 +128,7 @@ def test_autotuned_ensemble_matches_members_alone(oracle_lib):
     alone = [(Dycore(c.metrics, c.namelist), state_to_device(c.state)) for c in cases]
     batched = [(Dycore(c.metrics, c.namelist), state_to_device(c.state)) for c in cases]
     ens = Ensemble(batched, branches=2, autotune=True, trial_steps=1)
-    assert len(ens.tuned) == len(cases) and ens.tuned[2]["column_tile"] == -1  # moist: the column march
+    assert len(ens.tuned) == len(cases) and ens.tuned[2]["column_tile"] == -1  # moist: no LDS tile
     print(f"[batch] picks {ens.tuned}, trial {ens.batch_trial}", flush=True)
     for m, (c, (_, s)) in enumerate(zip(cases, batched)):  # tuning and the batch trial ran on copies
         _assert_bitwise(state_to_host(s), c.state, f"member {m} after tuning")

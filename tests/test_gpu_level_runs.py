@@ -5,7 +5,7 @@ across the waves of a workgroup instead of up one thread.  Covered: level counts
 last run one or two levels, one row and one column tile, column counts around a workgroup's 64,
 the deepest grid of the block forms and the first beyond them, the moist instances, and grids on
 both sides of the launch sizes at which the runs and the block forms stop (2048 waves; 512
-workgroups).  Every value is computed by the oracle's operations in the oracle's order, so the
+workgroups of k_rom, 256 of k_col_setup).  Every value is computed by the oracle's operations in the oracle's order, so the
 comparison is exact."""
 
 import numpy as np
@@ -20,7 +20,8 @@ SPECIES = ("qv", "qc", "qr", "qi", "qs", "qg")
 
 @pytest.mark.parametrize("grid,moist", [((4, 1, 4), False), ((64, 1, 5), False), ((65, 2, 9), True),
                                         ((63, 5, 21), False), ((30, 9, 63), True), ((30, 9, 64), False),
-                                        ((124, 256, 7), False), ((124, 257, 7), False), ((362, 361, 5), False),
+                                        ((124, 256, 7), False), ((124, 257, 7), False), ((62, 256, 5), False),
+                                        ((62, 257, 5), False), ((62, 256, 5), True), ((362, 361, 5), False),
                                         ((363, 363, 5), False)])
 def test_level_runs_match_oracle(oracle_lib, grid, moist):
     import torch

@@ -5,7 +5,7 @@ core/rk_addtend_dry.py:278, :359-360) and, with moist_adv_opt 1 or 2, are transp
 (runtime/operational_mode.py:3162-3316).  Covered: terrain with each moist_adv_opt, the
 2-D slab, the theta limiter and the species' limiter sharing their scratch on the final
 stage, the diffusions, a captured graph, wd_step_noalloc, and the autotuner (which must
-leave the caller's species untouched and keep the column march); every option at once
+leave the caller's species untouched and pick no LDS tile); every option at once
 (rotation, hypsometric_opt 2, both limiters, the filter); a state whose species are zero
 steps as the dry state; and the handle refuses mismatched states."""
 

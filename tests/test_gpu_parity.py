@@ -97,10 +97,10 @@ def test_bubble_64x64x40_100_steps(oracle_lib):
     _assert_parity(got, ref, case.state)
 
 
-@pytest.mark.parametrize("column", ["16x16", "8x16", "32x8", "16x8", "march"])
+@pytest.mark.parametrize("column", ["16x16", "8x16", "32x8", "16x8", "march", ""])
 def test_column_kernel_variants(oracle_lib, monkeypatch, column):
     """Every compiled form of the acoustic column kernel (tile shapes of the
-    LDS-tiled kernel and the column-march kernel) on a terrain case with the
+    LDS-tiled kernel, the column march and, by default, the column block) on a terrain case with the
     damping layer active, at the 50 levels of the 433x433x50 workload (the
     levels-per-thread instantiation it runs); the handle reads
     WRFDYN_COLUMN_TILE at creation."""

@@ -5,11 +5,11 @@ workgroups meeting at a grid barrier between phases.  Each virtual block is
 run by the same kernel code, with the block index, grid and thread layout of
 the standalone launch, as wd_step, so every member must come out bit for bit
 as that member stepped alone: FP64 and mixed, with rotation, at the uneven
-ensemble's member sizes, with members tuned to the LDS column tile, over
-several launches.  A barrier wait that runs out
-(forced here with a zero poll budget) must end every workgroup, be reported
-by wd_batch_status and leave the states as they were; the batch then steps
-normally.  Members the persistent step cannot run are refused.
+ensemble's member sizes, on the column block, held to the column march and
+tuned to the LDS column tile, over several launches.  A barrier wait that
+runs out (forced here with a zero poll budget) must end every workgroup, be
+reported by wd_batch_status and leave the states as they were; the batch then
+steps normally.  Members the persistent step cannot run are refused.
 """
 
 import numpy as np
@@ -70,6 +70,12 @@ def _dycore(case, precision, column=None):
             os.environ["WRFDYN_COLUMN_TILE"] = keep
 
 
+def _held_to(form, cases):
+    """_run_pair's arguments for a small ensemble on the column block (its default) or held to the march."""
+
+    return {"columns": [None if form == "block" else form] * len(cases), "expect_forms": [form] * len(cases)}
+
+
 def _run_pair(cases, steps, precision="fp64", columns=None, expect_kernels=None, remaps=None, expect_forms=None,
               alone_columns=None):
     """Each case stepped alone and in one persistent ensemble; returns both host states per case.
@@ -115,29 +121,37 @@ def _run_pair(cases, steps, precision="fp64", columns=None, expect_kernels=None,
     return out
 
 
-def test_persistent_members_match_individual_steps(oracle_lib):
+@pytest.mark.parametrize("form", ["block", "march"])
+def test_persistent_members_match_individual_steps(oracle_lib, form):
     cases = _small_cases()
-    out = _run_pair(cases, (1, 2))
+    out = _run_pair(cases, (1, 2), **_held_to(form, cases))
     ref = oracle_lib.run(cases[1].metrics, cases[1].namelist, cases[1].state, 3)
     errs = field_errors(out[1][1], ref)
     for k in FIELDS:
         assert errs[k] <= 1e-12, (k, errs[k])
 
 
-def test_persistent_mixed_members_match_individual_steps():
-    _run_pair(_small_cases()[:4], (2, 1), precision="mixed")
+@pytest.mark.parametrize("form", ["block", "march"])
+def test_persistent_mixed_members_match_individual_steps(form):
+    cases = _small_cases()[:4]
+    _run_pair(cases, (2, 1), precision="mixed", **_held_to(form, cases))
 
 
-def test_persistent_rotating_members_match_individual_steps():
+@pytest.mark.parametrize("form", ["block", "march"])
+def test_persistent_rotating_members_match_individual_steps(oracle_lib, form):
     cases = _small_cases()
     cases = [_rotating(cases[1], 45.0), cases[0], _rotating(cases[3], 30.0)]
-    _run_pair(cases, (2,))
+    out = _run_pair(cases, (2,), **_held_to(form, cases))
+    ref = oracle_lib.run(cases[0].metrics, cases[0].namelist, cases[0].state, 2)
+    errs = field_errors(out[0][1], ref)
+    for k in FIELDS:
+        assert errs[k] <= 1e-12, (k, errs[k])
 
 
 def test_persistent_runs_tuned_column_tiles(oracle_lib):
     """Members tuned to the 16x16 LDS column tile run it inside the launch at 1, 3 and 4 levels
     per thread (8, 40, 50 and 63 levels; the damping layer active at 50 and 63), beside a member
-    on the column march, one tuned to another tile shape and one too deep for the persistent
+    held to the column march, one tuned to another tile shape and one too deep for the persistent
     tile (64 levels), which both run as the column march.  Every member comes out bit for bit
     as stepped alone with its own choice; the 50-level tile member also against the oracle."""
 
@@ -154,7 +168,8 @@ def test_persistent_runs_tuned_column_tiles(oracle_lib):
         ic.stratified_terrain_3d(nx=17, ny=9, nz=64, **terrain),
     ]
     columns = ["16x16", "16x16", "16x16", "16x16", "march", "8x16", "16x16"]
-    out = _run_pair(cases, (2, 1), columns=columns, expect_kernels=[0, 0, 0, 0, -1, -1, -1])
+    out = _run_pair(cases, (2, 1), columns=columns, expect_kernels=[0, 0, 0, 0, -1, -1, -1],
+                    expect_forms=["tile"] * 4 + ["march"] * 3)
     ref = oracle_lib.run(cases[2].metrics, cases[2].namelist, cases[2].state, 3)
     errs = field_errors(out[2][1], ref)
     for k in FIELDS:
@@ -176,7 +191,7 @@ def test_persistent_column_tile_with_rotation_and_hardware_order():
 
 def test_persistent_autotune_keeps_the_faster_column_choice():
     """Ensemble(autotune=True, persistent=True): each member is tuned alone, then the persistent
-    step is timed with the members' tuned tiles and with every member on the column march, on
+    step is timed with the members' tuned tiles and with every member off its tile, on
     copies of the states, and the faster is kept.  The members' column kernels in the step follow
     that choice, the states are not touched by the trials, and every member is bit for bit as
     stepped alone."""
@@ -239,13 +254,23 @@ def test_set_tuned_config_round_trip_and_refusals():
     d.close()
 
 
-def test_persistent_mixed_form_keeps_the_column_march():
-    """The LDS column tile is FP64 only: a mixed-form member runs the column march."""
+@pytest.mark.parametrize("nz,column", [(40, "march"), (52, "16x16")])
+def test_persistent_mixed_form_keeps_the_column_march(nz, column):
+    """The LDS column tile is FP64 only: a mixed-form member held to the column march, or too deep
+    for the column block, runs the march whatever tile it was created with."""
 
     from wrf_gpu_amd import ic
 
+    cases = [ic.stratified_terrain_3d(nx=20, ny=18, nz=nz, dx=3000.0, u_sigma=1.0, sigma=0.5)]
+    _run_pair(cases, (2,), precision="mixed", columns=[column], expect_kernels=[-1], expect_forms=["march"])
+
+
+def test_persistent_mixed_form_runs_the_block_instead_of_a_tile():
+    from wrf_gpu_amd import ic
+
     cases = [ic.stratified_terrain_3d(nx=20, ny=18, nz=40, dx=3000.0, u_sigma=1.0, sigma=0.5)]
-    _run_pair(cases, (2,), precision="mixed", columns=["16x16"], expect_kernels=[-1])
+    _run_pair(cases, (2,), precision="mixed", columns=["16x16"], expect_kernels=[-1], expect_forms=["block"],
+              alone_columns=["march"])
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
