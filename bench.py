@@ -488,7 +488,7 @@ def ensemble_leg(steps: int, dev) -> dict:
                                            "members_on_column_tile": sum(k >= 0 for k in kernels)}
     ens.close()
     # the autotuned persistent step: members tuned alone, then the step timed with their tiles and with
-    # every member on the column march, the faster kept
+    # every member off its tile, the faster kept
     ens = Ensemble(members, persistent=True, autotune=True, trial_steps=1)
     ens.step(1)
     ens.status()

@@ -1,6 +1,6 @@
-// Acoustic small step (advance_uv, then the fused column kernel
-// advance_mu_t + advance_w + calc_p_rho) and the stage finish
-// (small_step_finish + grid%p refresh).
+// Acoustic small step (advance_uv, then advance_mu_t + advance_w + calc_p_rho
+// as the column block, the column march's two kernels or the LDS tile) and the
+// stage finish (small_step_finish + grid%p refresh).
 //
 // Each output value is computed with the reference's expression order; build
 // with -ffp-contract=off.
@@ -296,6 +296,10 @@ __device__ __forceinline__ void b_uv(const Blk& B, double* lds, DGrid g, DState 
   }
 }
 
+// Held to three waves a SIMD (168 VGPRs), which costs the PREP instance of the
+// runs two spilled registers; left to the compiler it runs at two: 195.2
+// against 198.5 us a launch at 433x433x50, 13.0 against 13.8 at 64x64x40 (but
+// 86 against 83 at 257x257x50).
 template <int BX, int BY, class TT, bool WET, bool PREP, bool RUNS>
 __global__ void __launch_bounds__(BX * BY) __attribute__((amdgpu_waves_per_eu(3))) k_uv(DGrid g, DState s, DWork w, double dts, int first, int kc) {
   __shared__ double sh[2][BY][7][BX];
@@ -1290,14 +1294,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 // each of its sweeps over the levels reads again what the sweep before it had
 // (dvdxi, omega, t_2ave, the phi rhs, the forward-swept w, theta, c2a, alt);
 // with a column's levels spread over the registers of a workgroup each array
-// is read once, 24 in all, and a small grid has thirteen times the waves.
+// is read once, 24 in all, and a 64x64x40 grid has 1408 waves (128 workgroups
+// of 11) where one column a thread gives it 64.
 // Four levels a wave is what 128 VGPRs (four waves per SIMD, one workgroup of
 // up to 16 waves per CU) hold without spilling; 7, 9 and 13 levels a wave at
 // 128, 168 and 256 VGPRs spilled and were slower (433x433x50: 14.8, 17.3 and
-// 14.3 ms a step against 13.3).  At 433x433x50 it moves 2.0 GB in 0.535 ms
-// (3.8 TB/s), bounded by HBM and by the loads that a workgroup cannot issue
-// before its sums; the march pair took 0.659 ms there and 0.144 ms at
-// 64x64x40, where the block takes 0.029.
+// 14.3 ms a step against 13.3).  At 433x433x50 it moves 2.0 GB in 0.520 ms
+// (3.9 TB/s), bounded by HBM and by the loads that a workgroup cannot issue
+// before its sums: a CU holds one workgroup, and one alone takes 29 us
+// (80x1x40).  The march pair takes 0.641 ms at 433x433x50 and 0.150 ms at
+// 64x64x40, the block 0.031 there.
 // ---------------------------------------------------------------------------
 constexpr int kBlockOwned = 62;   // columns owned per workgroup
 constexpr int kBlockExch = 7;     // values per wave and lane of the widest exchange
@@ -1692,7 +1698,8 @@ __global__ void __launch_bounds__(1024) k_column_block(DGrid g, DNamelist nl, DS
 // issued before the current level is computed.
 //
 // Where one column a thread leaves the GPU idle, a workgroup is 64 columns by
-// several waves, each marching a run of kc levels (64x64x40: 53 -> 9 us).  The
+// several waves, each marching a run of kc levels (64x64x40: 56 -> 17 us;
+// 310x160x40, 800 waves: 76 -> 66; 257x257x50, 1033 waves: 108 -> 116).  The
 // state is updated in place, so a wave reads the old ph of the level below
 // its run before the workgroup's barrier, after which the runs are stored.
 __device__ __forceinline__ void b_fin_col(const Blk& B, DGrid g, DState s, DState out, DWork w, int kc) {

@@ -110,7 +110,8 @@ struct DWork {
   // prep (3-D)
   double *u_work, *v_work, *w_work, *th_work, *ph_work;
   double *c2a, *alt, *pb, *ph1t, *php;  // ph1t = origin ph' + base ph (stage constant)
-  double *p, *al, *pm1;
+  double *p, *pm1;
+  double* al;  // null in a plain step: k_uv forms it (the adjoint's recompute stores it)
   // stage column setup
   double *rw_tend, *ph_tend, *ca, *calpha, *cgamma;
   // acoustic carried (ww: only levels 0 and nz carry between substeps)
@@ -216,13 +217,23 @@ inline int column_wave_levels(const DGrid& g, int n) {
 }
 // Kernels that hold a whole column in one workgroup, kBlockLevels w levels a
 // wave: the waves a grid of nz levels needs, 0 where a workgroup's 16 are too
-// few.
+// few.  k_column_block runs wherever it holds the levels: whole steps, march
+// -> block, 433 x 433 columns of 4, 8, 20, 30, 60 and 63 levels 1.07 -> 0.97,
+// 1.88 -> 1.70, 4.54 -> 4.10, 6.82 -> 5.71, 13.80 -> 12.18 and 14.51 -> 12.70
+// ms, 64 x 64 of 4, 20 and 63 levels 0.42 -> 0.35, 0.90 -> 0.50 and 2.19 ->
+// 0.84, 24 x 24 of 63 levels 1.90 -> 0.66, mixed and moist alike.  Only long
+// narrow grids lose, whose rows leave most of a workgroup's 62 columns empty:
+// 16x2000x50 4.18 -> 4.21, 4x4000x20 2.37 -> 2.92 ms.
 constexpr int kBlockLevels = 4;
-// The block form of k_rom pays while a launch has at most kFewBlocks workgroups
-// (two a CU), that of k_col_setup, which needs more of a CU, up to half of
-// them: 64x64x40 (64 and 128 workgroups) 23 -> 6.5 and 58 -> 32 us,
-// 141x123x45 (369) 26 -> 11 and 70 -> 77 us, 433x433x50 (3031) 49 -> 77 and
-// 228 -> 613 us, since a workgroup of one row shares no rows.
+// The block forms of k_rom and k_col_setup.  That of k_col_setup takes a CU's
+// registers (and spills some of its own at the 128 that 16 waves leave it), so
+// it pays up to one workgroup a CU: 38.5 us at 124x128x40 (256 workgroups);
+// from there on a second round starts, against the kernel of four rows a
+// workgroup, which shares their halo rows: 124x144x40 (288) 60.8 -> 67.2,
+// 141x123x45 (369) 68.0 -> 72.6, 433x433x50 (3031) 190 -> 577 us.  64x64x40
+// (128): 58 -> 32 us.  That of k_rom is kept to two a CU: 64x64x40 (64
+// workgroups) 23 -> 8.5, 141x123x45 (369) 26 -> 12.3 us; it would pay up to
+// 257x257x50 (1285: 35.2 -> 30.7 us), not at 433x433x50 (3031: 49 -> 77 us).
 constexpr unsigned kFewBlocks = 512;
 inline int column_block_waves(int nz) { return nz + 1 <= 16 * kBlockLevels ? (nz + kBlockLevels) / kBlockLevels : 0; }
 inline unsigned runs_of(int n, int kc) { return (unsigned)((n + kc - 1) / kc); }

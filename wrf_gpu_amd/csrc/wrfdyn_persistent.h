@@ -189,10 +189,15 @@ __device__ __forceinline__ void run_segment(const PSeg& S, const PMember& M, uns
 }
 
 // Column blocks of all members up to which the step runs them: two for each of
-// the 256 workgroups that fit with them (one a CU).  One 64x64x40 member (128
-// of them) takes 2.30 ms a step with the block and 3.36 ms with the march, whose
-// 64 waves leave the GPU idle; larger ensembles fill it and keep the march's
-// two workgroups a CU.
+// the 256 workgroups that fit with them (one a CU).  The march's 64 waves
+// leave the GPU idle there: march -> block, a step of 64x64x40 (128 blocks)
+// 3.36 -> 2.30 ms, 124x128x40 (256) 3.57 -> 2.40, 124x192x40 (384) 3.82 ->
+// 2.83, 124x256x40 (512) 4.31 -> 3.32, of 12 and 51 levels 2.27 -> 1.82 and
+// 5.19 -> 4.05 (64x64x8: 0.80 -> 0.82).  Large ensembles fill the GPU with the
+// march's two workgroups a CU: 310x320x40 (1600) 7.17 -> 8.17, four
+// members of 129 to 321 columns square (4402) 17.9 -> 22.2 ms; in between the
+// block would still win, 186x256x40 (768) 4.87 -> 4.21, 248x256x40 (1024) 5.58
+// -> 5.46.
 constexpr unsigned long long kPersistBlockTiles = 512;
 
 // s_waitcnt vmcnt(0) in the gfx9 encoding (vmcnt 0, expcnt 7, lgkmcnt 15):
@@ -269,7 +274,7 @@ __device__ __forceinline__ void step_phases(const PMember* __restrict__ members,
   }
 }
 
-// The step without the column tile (every member on the column march).
+// The step of members on the column march alone.
 template <bool MX>
 __global__ void __launch_bounds__(256) k_step_persistent(const PMember* __restrict__ members,
                                                         const PSeg* __restrict__ segs,
@@ -455,7 +460,7 @@ bool persistent_program(const std::vector<PMember>& members, const std::vector<i
     for (int it = 0; it < nsub[st]; ++it) {
       const int first = it == 0 ? 1 : 0;
       add_phase({{PK_UV, rk, first}});
-      // a member runs either the column-march pair or the LDS column tile
+      // a member runs the column-march pair, the column block or the LDS column tile
       add_phase({{PK_COLUMN_MU, rk, first}, {PK_COLUMN_BLOCK, rk, first}, {PK_COLUMN_TILE, rk, first}});
       if (any_march) add_phase({{PK_COLUMN_W, rk, first}});
     }

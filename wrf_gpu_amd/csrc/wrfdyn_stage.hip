@@ -1490,7 +1490,9 @@ __device__ __forceinline__ void b_col_setup(const Blk& B, double* lds, DGrid g, 
 // either side) and one wave per kBlockLevels levels: each wave forms its
 // levels' tendencies and matrix rows from its own loads, and the gamma
 // recurrence passes from wave to wave.  One wave more per four levels is what
-// a small grid lacks.
+// a small grid lacks (64x64x40: 58 -> 32 us).  At the 128 VGPRs that up to 16
+// waves a workgroup leave it, it spills 60 of them (68 moist, 56 mixed; about
+// 200 B of scratch a lane).
 template <class TT, bool WET>
 __global__ void __launch_bounds__(1024) k_col_setup_block(DGrid g, DNamelist nl, DState s, DWork w, double dts) {
   __shared__ double carry[64];
@@ -2404,8 +2406,8 @@ void launch_limiter(const DGrid& g, const DNamelist& nl, const DState& s, const 
 // the south v face; the raw cqw = (qtot(k) + qtot(k-1))/2 on w face k, 0 at
 // the surface and the lid.  k_tend_u/v scale the large-step PGF by cqu/cqv,
 // k_uv the acoustic one, k_col_setup forms rw_tend and the implicit-w
-// coefficients with cq1 = 1/(1 + cqw) and cq2 = cqw cq1, and k_column_w the
-// explicit part of the w equation with cq1.
+// coefficients with cq1 = 1/(1 + cqw) and cq2 = cqw cq1, and k_column_block
+// (or k_column_w) the explicit part of the w equation with cq1.
 // ---------------------------------------------------------------------------
 __device__ inline double qtot_at(const DState& s, size_t c) {
   return ((((s.q[0][c] + s.q[1][c]) + s.q[2][c]) + s.q[3][c]) + s.q[4][c]) + s.q[5][c];
